@@ -410,10 +410,14 @@ MemintArgs memint_args(const kb_ctx* c) {
   return a;
 }
 
-hipError_t launch_memint(int tile, unsigned grid, size_t lds, hipStream_t s, const MemintArgs* args,
+hipError_t launch_memint(int tile, unsigned grid, int maxN, hipStream_t s, const MemintArgs* args,
                          const int* wg_start, int nruns) {
+  // (a table of one run: its arguments are on the device only)
+  if (nruns > 1 && memint_runs_whole(tile, maxN))
+    return launch_memint_runs(MemintArgs{}, args, wg_start, nruns, grid, maxN, s);
   void* kargs[] = {(void*)&args, (void*)&wg_start, (void*)&nruns};
-  return hipLaunchKernel(kMemintVariants[tile].fn, dim3(grid), dim3(kMemintVariants[tile].threads), kargs, lds, s);
+  return hipLaunchKernel(kMemintVariants[tile].fn, dim3(grid), dim3(kMemintVariants[tile].threads), kargs,
+                         memint_lds(maxN), s);
 }
 
 size_t memint_lds(int N) { return sizeof(double) * 2 * (size_t)N * MB; }
@@ -427,19 +431,33 @@ int launch_hartree_step(kb_ctx* c) {
   return KB_OK;
 }
 
-// Split memory integral (orbit storage): partial sweeps over item ranges,
-// then the sums and the leapfrog, in the context's tile shape (the item
-// table in margs_dev has that shape's row height).
-int launch_memint_split(kb_ctx* c) {
-  const MemintVariant& v = kMemintVariants[c->tile];
-  const MemintArgs* margs = c->margs_dev;
-  int ns = c->msplit;
-  double* part = c->mpart;
-  void* kargs[] = {(void*)&margs, (void*)&ns, (void*)&part};
-  HIPCHK(c, hipLaunchKernel(v.partial, dim3(c->NB * c->msplit), dim3(v.threads), kargs, memint_lds(c->N), c->stream));
-  hipLaunchKernelGGL(memint_finish, dim3(c->NB), dim3(MEMINT_FINISH_THREADS), memint_lds(c->N), c->stream,
-                     c->margs_dev, c->msplit, c->mpart);
-  LAUNCHCHK(c);
+// The memory integral of the step in st_dev, in the context's tile shape
+// (the item table in margs_dev has that shape's row height).  Split form (few
+// site blocks): partial sweeps, then the sums and the leapfrog.
+int launch_memint_step(kb_ctx* c) {
+  const MemintArgs a = memint_args(c);
+  // (no integrals in the LO expansions: the leapfrog alone, in the item form)
+  const bool runs = a.integral && c->tile == 0 && c->rsplit > 1;
+  const bool whole = a.integral && memint_runs_whole(c->tile, c->N);
+  const int ns = runs ? c->rsplit : whole ? 1 : c->msplit;
+  if (ns > 1) {
+    if (runs) {
+      HIPCHK(c, launch_memint_runs_split(a, c->NB, ns, c->mpart, c->stream));
+    } else {
+      const MemintVariant& v = kMemintVariants[c->tile];
+      const MemintArgs* margs = c->margs_dev;
+      void* kargs[] = {(void*)&margs, (void*)&ns, (void*)&c->mpart};
+      HIPCHK(c, hipLaunchKernel(v.partial, dim3(c->NB * ns), dim3(v.threads), kargs, memint_lds(c->N), c->stream));
+    }
+    hipLaunchKernelGGL(memint_finish, dim3(c->NB), dim3(MEMINT_FINISH_THREADS), memint_lds(c->N), c->stream, a, ns,
+                       c->mpart);
+    LAUNCHCHK(c);
+    return KB_OK;
+  }
+  hipError_t e = whole
+                     ? launch_memint_runs(a, nullptr, nullptr, 1, c->NB, c->N, c->stream)
+                     : launch_memint(c->tile, c->NB, c->N, c->stream, c->margs_dev, c->wg0_dev, 1);
+  if (e != hipSuccess) return seterr(c, KB_ERR_HIP, "memory-integral launch failed: %s", hipGetErrorString(e));
   return KB_OK;
 }
 
@@ -462,12 +480,7 @@ int enqueue_step(kb_ctx* c) {
   }
   {
     StageTimer st(c, 0);
-    if (c->msplit > 1) {
-      if ((rc = launch_memint_split(c))) return rc;
-    } else {
-      hipError_t e = launch_memint(c->tile, c->NB, memint_lds(c->N), c->stream, c->margs_dev, c->wg0_dev, 1);
-      if (e != hipSuccess) return seterr(c, KB_ERR_HIP, "memory-integral launch failed: %s", hipGetErrorString(e));
-    }
+    if ((rc = launch_memint_step(c))) return rc;
   }
   return KB_OK;
 }
@@ -817,21 +830,26 @@ static int create_ctx(const kb_params* p, bool sym, kb_ctx** out) {
       return fail(KB_ERR_ARG);
     }
   }
-  // orbit storage leaves fewer site blocks than workgroup slots: split each
-  // block's memory integral over msplit workgroups, as many as fit the
-  // device's slots for this window's LDS size in one round (a grid that
-  // overfills some CUs by one workgroup waits for those CUs)
-  if (sym) {
-    int per_cu = 0;
-    hipDeviceProp_t prop;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)memint_partial<64, 2, 256>, 256,
-                                                     memint_lds(c->N)) != hipSuccess ||
-        hipGetDeviceProperties(&prop, p->device) != hipSuccess)
+  // few site blocks (orbit storage, 1D and small 2D lattices): split each
+  // block's memory integral over several workgroups.  In orbit storage every
+  // shape has a split form, with as many parts as fit the device's slots for
+  // this window's LDS size in one round (a grid that overfills some CUs by
+  // one workgroup waits for those CUs)
+  {
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, p->device) != hipSuccess ||
+        memint_runs_prepare() != hipSuccess)
       return fail(KB_ERR_HIP);
-    const int slots = per_cu * prop.multiProcessorCount;
-    c->msplit = std::max(1, std::min(KB_MSPLIT_MAX, slots / c->NB));
-    if (c->msplit > 1 &&
-        (rc = dmalloc(c, (void**)&c->mpart, (size_t)c->NB * c->msplit * 2 * c->N * MB * sizeof(double))))
+    if (sym) {
+      int per_cu = 0;
+      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)memint_partial<64, 2, 256>, 256,
+                                                       memint_lds(c->N)) != hipSuccess)
+        return fail(KB_ERR_HIP);
+      c->msplit = std::max(1, std::min(KB_MSPLIT_MAX, per_cu * cus / c->NB));
+    }
+    c->rsplit = memint_runs_split(0, c->N, c->NB, cus);
+    const int parts = std::max(c->msplit, c->rsplit);
+    if (parts > 1 && (rc = dmalloc(c, (void**)&c->mpart, (size_t)c->NB * parts * 2 * c->N * MB * sizeof(double))))
       return fail(rc);
   }
   if (hipMemsetAsync(c->H, 0, hcount * sizeof(double), c->stream) != hipSuccess) return fail(KB_ERR_HIP);
@@ -1410,10 +1428,7 @@ int kb_autotune(kb_ctx* c, int reps, int* best, double* ms) {
     // the steps use (split in orbit storage)
     for (int k = 0; k <= reps && rc == KB_OK; ++k) {
       if (k == 1 && hipEventRecord(a, c->stream) != hipSuccess) rc = seterr(c, KB_ERR_HIP, "autotune: event");
-      if (c->msplit > 1)
-        rc = launch_memint_split(c);
-      else if (launch_memint(v, c->NB, memint_lds(c->N), c->stream, c->margs_dev, c->wg0_dev, 1) != hipSuccess)
-        rc = seterr(c, KB_ERR_HIP, "autotune: launch failed");
+      if (rc == KB_OK) rc = launch_memint_step(c);
     }
     if (rc) break;
     float e_ms = 0.f;
@@ -1668,7 +1683,7 @@ int ens_enqueue(kb_ens* e) {
     }
     if (rc == KB_OK && e->lane_integrals && e->lwg[j] > 0) {
       // one shape for all members (their item tables follow its row height)
-      err = launch_memint(e->tile, e->lwg[j], memint_lds(e->lmaxN[j]), sj, e->margs_dev + e->lrun[j],
+      err = launch_memint(e->tile, e->lwg[j], e->lmaxN[j], sj, e->margs_dev + e->lrun[j],
                           e->lwg_dev + e->lrun[j], e->lrun[j + 1] - e->lrun[j]);
       if (err != hipSuccess) rc = ens_err(e, KB_ERR_HIP, "memint launch failed: %s", hipGetErrorString(err));
     }
@@ -1684,7 +1699,7 @@ int ens_enqueue(kb_ens* e) {
   }
   if (rc) return rc;
   if (!e->lane_integrals) {
-    err = launch_memint(e->tile, e->total_wg, memint_lds(e->maxN), e->stream, e->margs_dev, e->wg_dev, nr);
+    err = launch_memint(e->tile, e->total_wg, e->maxN, e->stream, e->margs_dev, e->wg_dev, nr);
     if (err != hipSuccess) return ens_err(e, KB_ERR_HIP, "memint launch failed: %s", hipGetErrorString(err));
   }
   return KB_OK;
@@ -1787,7 +1802,7 @@ int kb_ens_autotune(kb_ens* e, int reps, int* best, double* ms) {
     for (int k = 0; k <= reps && rc == KB_OK; ++k) {
       if (k == 1 && hipEventRecord(a, e->stream) != hipSuccess) rc = ens_err(e, KB_ERR_HIP, "autotune: event");
       if (rc == KB_OK &&
-          launch_memint(v, e->total_wg, memint_lds(e->maxN), e->stream, e->margs_dev, e->wg_dev, nr) != hipSuccess)
+          launch_memint(v, e->total_wg, e->maxN, e->stream, e->margs_dev, e->wg_dev, nr) != hipSuccess)
         rc = ens_err(e, KB_ERR_HIP, "autotune: launch failed");
     }
     if (rc) break;

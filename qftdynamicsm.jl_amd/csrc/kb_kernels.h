@@ -207,7 +207,18 @@ __global__ void memint_step(const MemintArgs* runs, const int* wg_start, int nru
 // them and runs the leapfrog (one run, grid = site blocks)
 template <int ROWS, int B, int TPB>
 __global__ void memint_partial(const MemintArgs* runs, int nsplit, double* part);
-__global__ void memint_finish(const MemintArgs* runs, int nsplit, const double* part);
+__global__ void memint_finish(MemintArgs a, int nsplit, const double* part);
+// The default shape (tile 0) as equal runs of the triangle's rows, in windows
+// that memint_runs_whole takes: one launch over `grid` site blocks of windows
+// up to N; a single run's arguments by value (nruns 1), or the tables of
+// memint_step.  The split form takes memint_runs_split(...) > 1 workgroups
+// per site block, followed by memint_finish.
+bool memint_runs_whole(int tile, int N);
+int memint_runs_split(int tile, int N, int NB, int cus);
+hipError_t memint_runs_prepare();
+hipError_t launch_memint_runs(const MemintArgs& one, const MemintArgs* runs, const int* wg_start, int nruns,
+                              unsigned grid, int N, hipStream_t s);
+hipError_t launch_memint_runs_split(const MemintArgs& a, int NB, int nsplit, double* part, hipStream_t s);
 
 // memory-integral tile shapes: ROWS slot rows per work item, B rows per
 // batch (two batches in flight), threads per workgroup; fn is the kernel

@@ -692,11 +692,11 @@ __global__ __launch_bounds__(TPB, 512 / TPB) void memint_partial(const MemintArg
   for (int i = tid; i < 2 * N * MB; i += blockDim.x) out[i] = smem[i];
 }
 
-// (1024 threads: the sum over the splits' partials is latency-bound)
-__global__ __launch_bounds__(MEMINT_FINISH_THREADS) void memint_finish(const MemintArgs* __restrict__ runs,
-                                                                       int nsplit, const double* __restrict__ part) {
+// (1024 threads, four partials in flight: the sum over the splits' partials
+// is latency-bound)
+__global__ __launch_bounds__(MEMINT_FINISH_THREADS) void memint_finish(MemintArgs a, int nsplit,
+                                                                       const double* __restrict__ part) {
   extern __shared__ double smem[];
-  const MemintArgs a = runs[0];
   const StepState ss = *a.st;
   const int N = a.N;
   double* accF = smem;
@@ -704,14 +704,362 @@ __global__ __launch_bounds__(MEMINT_FINISH_THREADS) void memint_finish(const Mem
   __shared__ double red[MEMINT_FINISH_THREADS / 64][MB];
   __shared__ double diagF[2][MB];
   const int mb = blockIdx.x;
-  const double* in = part + (size_t)mb * nsplit * 2 * N * MB;
-  for (int i = threadIdx.x; i < 2 * N * MB; i += blockDim.x) {
-    double v = 0.0;
-    for (int k = 0; k < nsplit; ++k) v += in[(size_t)k * 2 * N * MB + i];
-    smem[i] = v;
+  const size_t stride = (size_t)2 * N * MB;
+  const double* in = part + (size_t)mb * nsplit * stride;
+  for (int i = threadIdx.x; i < ss.Rmax * MB; i += blockDim.x) {
+    double f = 0.0, r = 0.0;
+    for (int k0 = 0; k0 < nsplit; k0 += 4) {
+      double x[4], y[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const double* q = in + min(k0 + u, nsplit - 1) * stride + i;
+        x[u] = q[0];
+        y[u] = q[N * MB];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        f += k0 + u < nsplit ? x[u] : 0.0;
+        r += k0 + u < nsplit ? y[u] : 0.0;
+      }
+    }
+    accF[i] = f;
+    accR[i] = r;
   }
   __syncthreads();
   memint_leapfrog(a, ss, mb, accF, accR, red, diagF);
+}
+
+// ---------------------------------------------------------------------------
+// The default shape in short windows, and wherever site blocks are few: the
+// same integrals with the triangle cut into equal runs.  The rows of the slot
+// triangle in use (4 slots each, in memory order: column block after column
+// block) are numbered, and every 8-lane worker of a site block takes one
+// contiguous run of them, crossing column blocks on the way.
+// Bound: HBM latency, not bandwidth -- a short window is a few KB to some 100
+// KB per site block.  The 64-row items gave 4 of 32 workers work at
+// N_mem = 16 and left a 64-row worker running alone at 96; runs of equal
+// length end together.  Small workgroups (one wave per site block up to
+// N_mem = 32, where rows t-1 and t-2 are also kept in LDS for the leapfrog)
+// put up to 16 site blocks on a CU, so one block's set-up and leapfrog hide
+// behind the others' loads.  The coefficients of a block are staged in LDS
+// while its first rows are on their way; one row (4 lines) is in flight per
+// worker: 2 or 3 need more than 128 registers, and fewer waves cost more
+// than the deeper pipeline gives.
+// Measured (64-row items -> runs): 112^3 N_mem = 16 4868 -> 906 us (0.63 ->
+// 3.4 TB/s), 64^3 N_mem = 32 1267 -> 544 us, 48^3 N_mem = 48 742 -> 466 us,
+// 42^3 N_mem = 96 1146 -> 1085 us (5.1 TB/s), 32^3 N_mem = 150 1111 -> 1043
+// us (5.7 TB/s), 16^3 N_mem = 64 37.6 -> 30.6 us, 16^2 N_mem = 24 13.3 -> 6.4
+// us.  Past N_mem = 208 the staged items are as fast (32^3 N_mem = 300: 3840
+// against 3842-3988 us) and keep the call.
+// ---------------------------------------------------------------------------
+__host__ __device__ inline int run_base(int J, int R) { return J * R - CB / 2 * J * (J - 1); }
+__host__ __device__ inline int run_rows(int R) { return run_base((R + CB - 1) / CB, R); }
+
+// column block of row number g < run_rows(R): the largest J with
+// run_base(J, R) <= g (a root in float, corrected by at most one)
+__device__ __forceinline__ int run_block(int g, int R) {
+  const float h = (float)(R + CB / 2);
+  int J = (int)((h - sqrtf(fmaxf(h * h - 2.0f * CB * (float)g, 0.0f))) * (1.0f / CB));
+  J = max(0, min(J, (R - 1) / CB));
+  while (J > 0 && run_base(J, R) > g) --J;
+  while (CB * (J + 1) < R && run_base(J + 1, R) <= g) ++J;
+  return J;
+}
+
+// offset in doubles of slot pair (a, b) from the site block's first pair
+__device__ __forceinline__ int pair_rel(int a, int b, int N) {
+  const int hi = max(a, b), lo = min(a, b);
+  const int J = lo / CB;
+  return (CB * (N * J - CB / 2 * J * (J - 1)) + (hi - J * CB) * CB + (lo - J * CB)) * (2 * MB);
+}
+
+// Sweep of one site block by worker w of nw: cf (v, ms per slot and lane) and
+// the accumulators are staged by the whole workgroup, the first rows are on
+// their way meanwhile.
+template <int D, bool STASH>
+__device__ __forceinline__ void memint_runs(const MemintArgs& a, const StepState& ss, int mb, double2* cf,
+                                            double* accF, double* accR, double2* rows, int w, int nw) {
+  const int N = a.N, R = ss.Rmax, smin = ss.s_min;
+  const int tid = threadIdx.x, lane = tid & (MB - 1);
+  const int T = a.integral ? run_rows(R) : 0;
+  const int g0 = T * w / nw, n = T * (w + 1) / nw - g0;
+  int J = 0, r = 0;
+  double2 e[D][CB];
+  const double* p = a.H + hoff(mb, 0, lane, a.NP);
+  const int gap = (N - R) * (CB * 2 * MB);  // rows not in use at the end of a column block
+  int rp = 0, cp = 0, k = 0;  // next row to fetch, its column block's first slot
+  auto fetch = [&](double2 (&b)[CB]) {
+#pragma unroll
+    for (int jc = 0; jc < CB; ++jc) b[jc] = ld_stream(p + jc * 2 * MB);
+    if (++k < n) {  // past the last row of the run: read it again
+      p += CB * 2 * MB;
+      if (++rp == R) {
+        cp += CB;
+        rp = cp;
+        p += gap;
+      }
+    }
+  };
+  if (n > 0) {
+    J = run_block(g0, R);
+    r = CB * J + g0 - run_base(J, R);
+    rp = r;
+    cp = CB * J;
+    p += (CB * (N * J - CB / 2 * J * (J - 1)) + (r - CB * J) * CB) * (2 * MB);
+#pragma unroll
+    for (int d = 0; d < D; ++d) fetch(e[d]);
+  }
+  for (int x = tid >> 3; x < R; x += blockDim.x >> 3) {
+    const double2 fs = ld_global(a.S + soff(mb, x, lane, N));
+    double wt, m;
+    slot_weights(x, smin, N, ss.L, wt, m);
+    cf[x * MB + lane] = x == ss.dead ? make_double2(0.0, 0.0) : make_double2(wt * fs.x, m * fs.y);
+    accF[x * MB + lane] = 0.0;
+    accR[x * MB + lane] = 0.0;
+  }
+  __syncthreads();
+  if (n > 0) {
+    // column slots c0 .. c0 + 3: u, v and the sums.  ms is only needed where
+    // time order is reversed (c < smin), and there u = ms.
+    double uc[CB], vc[CB], cF[CB], cR[CB];
+    unsigned phi = 0;  // bit jc: column slot lies before smin
+    auto columns = [&](int c0) {
+      phi = 0;
+#pragma unroll
+      for (int jc = 0; jc < CB; ++jc) {
+        const int c = c0 + jc;
+        const double2 q = c < R ? cf[c * MB + lane] : make_double2(0.0, 0.0);
+        vc[jc] = q.x;
+        uc[jc] = c == smin ? 0.5 * q.y : q.y;
+        cF[jc] = cR[jc] = 0.0;
+        phi |= (c < smin ? 1u : 0u) << jc;
+      }
+    };
+    auto flush = [&](int c0) {
+#pragma unroll
+      for (int jc = 0; jc < CB; ++jc)
+        if (c0 + jc < R) {
+          atomicAdd(&accF[(c0 + jc) * MB + lane], cF[jc]);
+          atomicAdd(&accR[(c0 + jc) * MB + lane], cR[jc]);
+        }
+    };
+    int c0 = CB * J;
+    columns(c0);
+    int left = n;
+    auto use = [&](double2 (&b)[CB]) {
+      const double2 q = cf[r * MB + lane];
+      const double ur = r == smin ? 0.5 * q.y : q.y;
+      const unsigned neg = r >= smin ? phi : 0u;
+      double rowF = 0.0, rowR = 0.0;
+      if constexpr (STASH) {
+        // rows t-1 and t-2 for the leapfrog: slot pairs with s_tm1 or s_tm2
+        const int d1 = ss.s_tm1 - c0, d2 = ss.s_tm2 - c0;
+        if (r == ss.s_tm1 || r == ss.s_tm2) {
+          double2* o = rows + (r == ss.s_tm1 ? 0 : N * MB) + c0 * MB + lane;
+#pragma unroll
+          for (int jc = 0; jc < CB; ++jc)
+            if (c0 + jc <= r) o[jc * MB] = b[jc];
+        }
+#pragma unroll
+        for (int jc = 0; jc < CB; ++jc) {
+          if (d1 == jc && c0 + jc <= r) rows[r * MB + lane] = b[jc];
+          if (d2 == jc && c0 + jc <= r) rows[(N + r) * MB + lane] = b[jc];
+        }
+      }
+      if (__any(r < c0 + CB)) {
+        // a worker is on its block's diagonal, which feeds its row once; the
+        // slots above it are padding
+#pragma unroll
+        for (int jc = 0; jc < CB; ++jc) {
+          if (c0 + jc == r) rowF -= ur * b[jc].x;
+          if (c0 + jc >= r) b[jc] = make_double2(0.0, 0.0);
+        }
+      }
+#pragma unroll
+      for (int jc = 0; jc < CB; ++jc) {
+        const bool nf = (neg >> jc) & 1u;
+        rowF -= uc[jc] * b[jc].x + (nf ? 0.0 : vc[jc]) * b[jc].y;
+        rowR += (nf ? uc[jc] : 0.0) * b[jc].y;
+        cF[jc] += (nf ? q.x : 0.0) * b[jc].y - ur * b[jc].x;
+        cR[jc] -= (nf ? 0.0 : q.y) * b[jc].y;
+      }
+      atomicAdd(&accF[r * MB + lane], rowF);
+      atomicAdd(&accR[r * MB + lane], rowR);
+      if (++r == R) {
+        flush(c0);
+        c0 += CB;
+        r = c0;
+        if (c0 < R) columns(c0);
+      }
+    };
+    bool more = true;
+    while (more) {
+#pragma unroll
+      for (int d = 0; d < D; ++d)
+        if (more) {
+          use(e[d]);
+          more = --left > 0;
+          fetch(e[d]);
+        }
+    }
+    if (c0 < R) flush(c0);
+  }
+  __syncthreads();
+}
+
+// memint_leapfrog with the coefficients in LDS; red: a row of MB doubles per wave
+template <int TPB, bool STASH>
+__device__ __forceinline__ void leapfrog_runs(const MemintArgs& a, const StepState& ss, int mb, const double2* cf,
+                                              const double* accF, const double* accR, const double2* rows,
+                                              double (*red)[MB], double (*diagF)[MB]) {
+  constexpr int NW = TPB / MB;
+  constexpr int LU = 4;  // slots per worker in flight
+  const int N = a.N, R = ss.Rmax, smin = ss.s_min;
+  const int tid = threadIdx.x, lane = tid & (MB - 1), worker = tid >> 3;
+  const int p = mb * MB + lane;
+  const bool real_site = p < a.V;
+  const double dt = a.dt, dt2 = dt * dt, dt3 = dt * dt * dt;
+  const double Om = (a.kL2[p] + a.m2[0]) * dt2;  // setomega2values!, Evolution.jl:918-921
+  double dsum = 0.0;
+  double* __restrict__ Hw = a.H + hoff(mb, 0, lane, a.NP);
+  for (int x0 = worker; x0 < R; x0 += NW * LU) {
+    double2 e1[LU], e2[LU];
+#pragma unroll
+    for (int u = 0; u < LU; ++u) {
+      const int x = min(x0 + u * NW, R - 1);
+      if (STASH && a.integral) {
+        e1[u] = rows[x * MB + lane];
+        e2[u] = rows[(N + x) * MB + lane];
+      } else {
+        e1[u] = ld_global(Hw + pair_rel(ss.s_tm1, x, N));
+        e2[u] = ld_global(Hw + pair_rel(ss.s_tm2, x, N));
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < LU; ++u) {
+      const int x = x0 + u * NW;
+      if (x >= R || x == ss.dead) continue;
+      const int tx = ss.tmin + window_pos(x, smin, N);
+      const double r1 = e1[u].y * (ss.s_tm1 >= x ? 1.0 : -1.0);
+      const double r2 = e2[u].y * (ss.s_tm2 >= x ? 1.0 : -1.0);
+      const double Fn = (2.0 - Om) * e1[u].x - e2[u].x + accF[x * MB + lane] * dt3;
+      const double rn = tx == ss.t - 1 ? dt : (2.0 - Om) * r1 - r2 + accR[x * MB + lane] * dt3;
+      if (real_site)
+        *reinterpret_cast<double2*>(Hw + pair_rel(ss.s_t, x, N)) = make_double2(Fn, rn * (ss.s_t >= x ? 1.0 : -1.0));
+      // terms of getRHS_F!(t,t) (Evolution.jl:973) over the fresh row
+      if (a.integral) {
+        const double2 q = cf[x * MB + lane];
+        dsum += -(x == smin ? 0.5 * q.y : q.y) * Fn - q.x * rn;
+      }
+      if (tx == ss.t - 1) diagF[0][lane] = Fn;
+      if (tx == ss.t - 2) diagF[1][lane] = Fn;
+    }
+  }
+  dsum += __shfl_xor(dsum, 8);
+  dsum += __shfl_xor(dsum, 16);
+  dsum += __shfl_xor(dsum, 32);
+  if ((tid & 63) < MB) red[tid >> 6][lane] = dsum;
+  __syncthreads();
+  if (tid < MB) {
+    double RF = 0.0;
+#pragma unroll
+    for (int wv = 0; wv < TPB / 64; ++wv) RF += red[wv][tid];
+    const double Ftt = (2.0 - Om) * diagF[0][tid] - diagF[1][tid] + RF * dt3;
+    if (real_site)
+      *reinterpret_cast<double2*>(Hw + pair_rel(ss.s_t, ss.s_t, N)) = make_double2(Ftt, 0.0);
+  }
+}
+
+// One workgroup per site block; a single run's arguments come by value (no
+// chain of loads before the first row), those of several runs from a table.
+template <int D, int TPB, bool STASH>
+__global__ __launch_bounds__(TPB, D > 1 ? 3 : 4) void memint_step_runs(MemintArgs one,
+                                                                       const MemintArgs* __restrict__ runs,
+                                                                       const int* __restrict__ wg_start, int nruns) {
+  extern __shared__ double smem[];
+  MemintArgs a = one;
+  int mb = blockIdx.x;
+  if (nruns > 1) {
+    int run = 0;
+    while (run + 1 < nruns && (int)blockIdx.x >= wg_start[run + 1]) ++run;
+    a = runs[run];
+    mb -= wg_start[run];
+  }
+  const StepState ss = *a.st;
+  double2* cf = reinterpret_cast<double2*>(smem);
+  double* accF = smem + 2 * a.N * MB;
+  double* accR = accF + a.N * MB;
+  double2* rows = reinterpret_cast<double2*>(accR + a.N * MB);  // STASH: rows t-1, t-2
+  __shared__ double red[TPB / 64][MB];
+  __shared__ double diagF[2][MB];
+  memint_runs<D, STASH>(a, ss, mb, cf, accF, accR, rows, threadIdx.x >> 3, TPB / MB);
+  leapfrog_runs<TPB, STASH>(a, ss, mb, cf, accF, accR, rows, red, diagF);
+}
+
+// Split form: the runs of a site block over the workers of nsplit
+// workgroups, whose accumulators go to part; memint_finish does the rest.
+template <int D, int TPB>
+__global__ __launch_bounds__(TPB, D > 1 ? 3 : 4) void memint_partial_runs(MemintArgs a, int nsplit,
+                                                                          double* __restrict__ part) {
+  extern __shared__ double smem[];
+  const StepState ss = *a.st;
+  const int N = a.N, R = ss.Rmax;
+  const int mb = blockIdx.x / nsplit, sp = blockIdx.x - mb * nsplit;
+  double2* cf = reinterpret_cast<double2*>(smem);
+  double* accF = smem + 2 * N * MB;
+  double* accR = accF + N * MB;
+  memint_runs<D, false>(a, ss, mb, cf, accF, accR, nullptr, sp * (TPB / MB) + ((int)threadIdx.x >> 3),
+                        nsplit * (TPB / MB));
+  double* out = part + (size_t)blockIdx.x * 2 * N * MB;
+  for (int i = threadIdx.x; i < R * MB; i += TPB) {
+    out[i] = accF[i];
+    out[N * MB + i] = accR[i];
+  }
+}
+
+constexpr int RUNS_MAX_N = 208;       // longest window of the whole-block form
+constexpr int RUNS_SPLIT_MIN_N = 48;  // shorter windows: the second launch costs more than it gives
+constexpr int RUNS_SPLIT_MAX_N = 600; // 256 bytes of LDS per slot
+constexpr int RUNS_SPLIT_THREADS = 512;
+
+bool memint_runs_whole(int tile, int N) { return tile == 0 && N <= RUNS_MAX_N; }
+
+// Workgroups per site block: one per CU in all.  16^2 and 1D lattices, and
+// orbit storage, have fewer site blocks than CUs: 128 sites in 1D at
+// N_mem = 400 took 298 us on 16 CUs and take 54 us on 256; 122 blocks
+// (32^3 in orbits) 247 us as 6 parts of 256 threads and 215 us as 2 of 512.
+int memint_runs_split(int tile, int N, int NB, int cus) {
+  if (tile != 0 || N < RUNS_SPLIT_MIN_N || N > RUNS_SPLIT_MAX_N) return 1;
+  return max(1, min(16, cus / NB));
+}
+
+hipError_t memint_runs_prepare() {
+  return hipFuncSetAttribute((const void*)memint_partial_runs<3, RUNS_SPLIT_THREADS>,
+                             hipFuncAttributeMaxDynamicSharedMemorySize, RUNS_SPLIT_MAX_N * 32 * MB);
+}
+
+// Threads per site block: a wave up to N_mem = 32 and two up to 192, if the
+// blocks fill the CUs that way (2048 of them); four otherwise, and eight for
+// long windows on fewer than two blocks per CU (256 blocks, N_mem = 200: 149
+// us at 256 threads, 121 at 512).
+hipError_t launch_memint_runs(const MemintArgs& one, const MemintArgs* runs, const int* wg_start, int nruns,
+                              unsigned grid, int N, hipStream_t s) {
+  const size_t lds = sizeof(double) * 4 * (size_t)N * MB;
+  if (grid >= 2048 && N <= 32)
+    hipLaunchKernelGGL((memint_step_runs<1, 64, true>), dim3(grid), dim3(64), 2 * lds, s, one, runs, wg_start, nruns);
+  else if (grid >= 2048 && N <= 192)
+    hipLaunchKernelGGL((memint_step_runs<1, 128, false>), dim3(grid), dim3(128), lds, s, one, runs, wg_start, nruns);
+  else if (grid >= 512 || N < 128)
+    hipLaunchKernelGGL((memint_step_runs<1, 256, false>), dim3(grid), dim3(256), lds, s, one, runs, wg_start, nruns);
+  else
+    hipLaunchKernelGGL((memint_step_runs<3, 512, false>), dim3(grid), dim3(512), lds, s, one, runs, wg_start, nruns);
+  return hipGetLastError();
+}
+
+hipError_t launch_memint_runs_split(const MemintArgs& a, int NB, int nsplit, double* part, hipStream_t s) {
+  hipLaunchKernelGGL((memint_partial_runs<3, RUNS_SPLIT_THREADS>), dim3(NB * nsplit), dim3(RUNS_SPLIT_THREADS),
+                     sizeof(double) * 4 * (size_t)a.N * MB, s, a, nsplit, part);
+  return hipGetLastError();
 }
 
 // the tile shapes the autotuner chooses from, as the whole-block kernel and
