@@ -4,12 +4,15 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <exception>
 #include <new>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../include/qftkb.h"
@@ -490,11 +493,86 @@ int upload(kb_ctx* c, double* dst, const double* src, size_t n) {
   return KB_OK;
 }
 
-int download(kb_ctx* c, double* dst, const double* src, size_t n) {
-  HIPCHK(c, hipMemcpyAsync(dst, src, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+// Device arrays of n doubles into caller arrays, through the context's pinned
+// memory.  What fits it goes in one copy.  Larger arrays go in halves of it,
+// the next half's copy running while HOST_COPY_THREADS threads write the
+// previous one out: the caller's fresh pages cost a single thread more time
+// than the copy.
+constexpr int HOST_COPY_THREADS = 6;
+
+int download_many(kb_ctx* c, int narr, double* const* dst, const double* const* src, size_t n) {
+  struct Piece {
+    double* d;
+    const double* s;
+    size_t n;
+  };
+  const size_t half = c->hstage_n / 2;
+  if (n * narr <= c->hstage_n) {
+    for (int k = 0; k < narr; ++k)
+      HIPCHK(c, hipMemcpyAsync(c->hdata + k * n, src[k], n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    for (int k = 0; k < narr; ++k) std::memcpy(dst[k], c->hdata + k * n, n * sizeof(double));
+    return KB_OK;
+  }
+  std::vector<Piece> pieces;
+  for (int k = 0; k < narr; ++k)
+    for (size_t o = 0; o < n; o += half) pieces.push_back({dst[k] + o, src[k] + o, std::min(half, n - o)});
+  const int np = (int)pieces.size();
+  // pieces handed out (-1: stop), their threads, and the shares of the last
+  // one that are not written yet
+  std::atomic<int> ready{0}, workers{0}, left{0};
+  std::vector<std::thread> pool;
+  auto share = [&](int p, int i, int of) {
+    const Piece& q = pieces[p];
+    const size_t b = q.n * i / of, e = q.n * (i + 1) / of;
+    std::memcpy(q.d + b, c->hdata + (p & 1) * half + b, (e - b) * sizeof(double));
+  };
+  auto work = [&](int i) {
+    for (int p = 0; p < np; ++p) {
+      int r;
+      while ((r = ready.load(std::memory_order_acquire)) <= p) {
+        if (r < 0) return;
+        std::this_thread::yield();
+      }
+      share(p, i, workers.load(std::memory_order_relaxed));
+      left.fetch_sub(1, std::memory_order_release);
+    }
+  };
+  try {
+    pool.reserve(HOST_COPY_THREADS);
+    for (int i = 0; i < HOST_COPY_THREADS; ++i) pool.emplace_back(work, i);
+  } catch (const std::exception&) {
+    // as many threads as there are; with none this thread copies
+  }
+  const int nw = (int)pool.size();
+  workers.store(nw, std::memory_order_relaxed);
+  auto drain = [&] {
+    while (left.load(std::memory_order_acquire) > 0) std::this_thread::yield();
+  };
+  hipError_t err = hipSuccess;
+  for (int p = 0; p < np; ++p) {
+    // into the half that piece p - 2 left: it was drained before piece p - 1
+    // was handed out
+    err = hipMemcpyAsync(c->hdata + (p & 1) * half, pieces[p].s, pieces[p].n * sizeof(double), hipMemcpyDeviceToHost,
+                         c->stream);
+    if (err == hipSuccess) err = hipStreamSynchronize(c->stream);
+    if (err != hipSuccess) break;
+    drain();
+    if (nw) {
+      left.store(nw, std::memory_order_relaxed);
+      ready.store(p + 1, std::memory_order_release);
+    } else {
+      share(p, 0, 1);
+    }
+  }
+  drain();
+  if (err != hipSuccess) ready.store(-1, std::memory_order_release);
+  for (auto& t : pool) t.join();
+  HIPCHK(c, err);
   return KB_OK;
 }
+
+int download(kb_ctx* c, double* dst, const double* src, size_t n) { return download_many(c, 1, &dst, &src, n); }
 
 int lat_upload(kb_ctx* c, double* dst, const double* src) {
   if (!c->sym) return upload(c, dst, src, c->V);
@@ -507,6 +585,14 @@ int lat_upload(kb_ctx* c, double* dst, const double* src) {
 
 int lat_download(kb_ctx* c, double* dst, const double* src) {
   if (!c->sym) return download(c, dst, src, c->V);
+  if ((size_t)c->Vl <= c->hstage_n) {
+    hipLaunchKernelGGL(expand_kernel, dim3((c->Vl + 255) / 256), dim3(256), 0, c->stream, src, c->V, c->smap_dev,
+                       c->Vl, 1, c->hdata);
+    LAUNCHCHK(c);
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    std::memcpy(dst, c->hdata, sizeof(double) * c->Vl);
+    return KB_OK;
+  }
   c->lat_tmp.resize(c->V);
   int rc = download(c, c->lat_tmp.data(), src, c->V);
   if (rc) return rc;
@@ -514,17 +600,26 @@ int lat_download(kb_ctx* c, double* dst, const double* src) {
   return KB_OK;
 }
 
+// where a kernel puts one lattice of stored sites for the caller, and its way
+// from there: full storage writes pinned host memory where it fits
+double* lattice_out(kb_ctx* c) { return !c->sym && (size_t)c->V <= c->hstage_n ? c->hdata : c->vbuf; }
+
+int deliver(kb_ctx* c, double* dst, const double* from) {
+  if (from != c->hdata) return lat_download(c, dst, from);
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  std::memcpy(dst, from, sizeof(double) * c->V);
+  return KB_OK;
+}
+
 void drop_graph(kb_ctx* c);
 
 void free_all(kb_ctx* c) {
   drop_graph(c);
-  for (void* ptr : {(void*)c->H, (void*)c->S, (void*)c->W, (void*)c->kL2, (void*)c->m2, (void*)c->hpart, (void*)c->partial,
-                    (void*)c->modes, (void*)c->vbuf, (void*)c->tw, (void*)c->flag, (void*)c->items_r[0],
-                    (void*)c->items_r[1], (void*)c->items_r[2], (void*)c->smap_dev, (void*)c->rmap_dev,
-                    (void*)c->wgt_dev, (void*)c->PF, (void*)c->PR, (void*)c->IR, (void*)c->Iring, (void*)c->Xn,
-                    (void*)c->stfill_dev, (void*)c->pitems, (void*)c->mpart, (void*)c->npart, (void*)c->ncv, (void*)c->Mo, (void*)c->Yo, (void*)c->Xo, (void*)c->G,
-                    (void*)c->st_dev, (void*)c->stptr_dev, (void*)c->N_dev, (void*)c->margs_dev, (void*)c->wg0_dev})
+  for (void* ptr : {(void*)c->H, (void*)c->S, (void*)c->W, (void*)c->PF, (void*)c->PR, (void*)c->IR, (void*)c->Iring,
+                    (void*)c->Xn, (void*)c->stfill_dev, (void*)c->pitems, (void*)c->mpart, (void*)c->npart,
+                    (void*)c->ncv, (void*)c->Mo, (void*)c->Yo, (void*)c->Xo, (void*)c->G, c->arena})
     if (ptr) (void)hipFree(ptr);
+  if (c->hstage) (void)hipHostFree(c->hstage);
   adj_free(c);
   for (int s = 0; s < NSTAGE; ++s)
     for (auto& ev : c->pending[s]) {
@@ -544,8 +639,6 @@ int dmalloc(kb_ctx* c, void** ptr, size_t bytes) {
   c->bytes += bytes;
   return KB_OK;
 }
-
-int meas_grid(const kb_ctx* c) { return (c->V + MEAS_THREADS - 1) / MEAS_THREADS; }
 
 // The plane kernels' workspace: W holds one complex lattice per row between
 // the passes (3D lattices, and the pencil passes past Nx = 64); Xn keeps the
@@ -712,20 +805,6 @@ static int create_ctx(const kb_params* p, bool sym, kb_ctx** out) {
     if (hipMemcpy(c->pitems, items.data(), sizeof(int2) * items.size(), hipMemcpyHostToDevice) != hipSuccess)
       return fail(KB_ERR_HIP);
   }
-  if (sym) {
-    std::vector<int> rmap(c->Vl, -1);
-    std::vector<double> wgt(c->V, 0.0);
-    for (int s = 0; s < c->Vl; ++s) wgt[c->orbit_of[s]] += 1.0;
-    for (int r = 0; r < c->V; ++r) rmap[c->rep_site[r]] = r;
-    if ((rc = dmalloc(c, (void**)&c->smap_dev, sizeof(int) * c->Vl)) ||
-        (rc = dmalloc(c, (void**)&c->rmap_dev, sizeof(int) * c->Vl)) ||
-        (rc = dmalloc(c, (void**)&c->wgt_dev, sizeof(double) * c->V)))
-      return fail(rc);
-    if (hipMemcpy(c->smap_dev, c->orbit_of.data(), sizeof(int) * c->Vl, hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(c->rmap_dev, rmap.data(), sizeof(int) * c->Vl, hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(c->wgt_dev, wgt.data(), sizeof(double) * c->V, hipMemcpyHostToDevice) != hipSuccess)
-      return fail(KB_ERR_HIP);
-  }
   // orbit storage, LambdaNLO: the self-energy stage as products with the
   // orbit cosine matrix Mo[o][b] = sum_{x in orbit b} cos(2 pi k_o . x / Nx),
   // k_o the representative of orbit o (zero-padded to the product's tiles)
@@ -768,47 +847,98 @@ static int create_ctx(const kb_params* p, bool sym, kb_ctx** out) {
     c->fft_tile = KB_FFT_ORBIT_PRODUCT;
   }
   if (c->fft_tile != KB_FFT_ORBIT_PRODUCT && (rc = ensure_plane_workspace(c))) return fail(rc);
-  if ((rc = dmalloc(c, (void**)&c->kL2, (size_t)c->Vpad * sizeof(double)))) return fail(rc);
-  if ((rc = dmalloc(c, (void**)&c->m2, 8 * sizeof(double)))) return fail(rc);
-  if ((rc = dmalloc(c, (void**)&c->hpart, hartree_part_doubles(c->V) * sizeof(double)))) return fail(rc);
-  if ((rc = dmalloc(c, (void**)&c->partial, (size_t)6 * meas_grid(c) * sizeof(double)))) return fail(rc);
+  c->hstage_n = std::max((size_t)6 * c->Vl, (size_t)4 * c->N);
+  if (c->hstage_n > HSTAGE_MAX) c->hstage_n = 2 * HSTAGE_MAX;
+  // The small buffers live in one allocation: first those with initial
+  // values, copied from a host image in one transfer (a context of a small
+  // lattice spent most of its creation on some thirty allocations and copies)
+  {
+    struct Part {
+      void** ptr;
+      size_t off;
+    };
+    std::vector<Part> parts;
+    std::vector<char> image;
+    size_t used = 0;
+    auto place = [&](void** ptr, size_t bytes) {
+      parts.push_back({ptr, used});
+      used += (std::max(bytes, size_t(8)) + 255) / 256 * 256;
+    };
+    auto with = [&](void** ptr, const void* src, size_t bytes) {  // src NULL: zeros
+      const size_t off = used;
+      place(ptr, bytes);
+      image.resize(used, 0);
+      if (src) std::memcpy(image.data() + off, src, bytes);
+    };
+    std::vector<double2> tw(p->Nx);  // exp(-2 pi i k / Nx)
+    fft_twiddles(p->Nx, tw.data());
+    std::vector<double> k2(c->Vpad, 0.0), k1(p->Nx);  // the default k^2 table
+    for (int nd = 0; nd < p->Nx; ++nd) {
+      const double s = std::sin(M_PI * (double)nd / (double)p->Nx);
+      k1[nd] = 4.0 * s * s;
+    }
+    for (int i = 0; i < c->V; ++i) {
+      int rem = sym ? c->rep_site[i] : i;
+      double s2 = 0.0;
+      for (int d = 0; d < p->sdim; ++d) {
+        s2 += k1[rem % p->Nx];
+        rem /= p->Nx;
+      }
+      k2[i] = s2;
+    }
+    with((void**)&c->kL2, k2.data(), sizeof(double) * c->Vpad);
+    with((void**)&c->tw, tw.data(), sizeof(double2) * p->Nx);
+    // memory-integral work items: chunks of MEMINT_ROWS rows of each column
+    // block, in storage order
+    for (int i = 0; i < 3; ++i) {
+      const int rows = MEMINT_ROW_CHOICES[i];
+      std::vector<int2> items;
+      for (int J = 0; J * CB < c->N; ++J)
+        for (int k = 0; J * CB + k * rows < c->N; ++k) items.push_back(make_int2(J, k));
+      c->nitems_r[i] = (int)items.size();
+      with((void**)&c->items_r[i], items.data(), sizeof(int2) * items.size());
+      if (rows == MEMINT_ROWS) c->nitems = c->nitems_r[i];
+    }
+    if (sym) {
+      std::vector<int> rmap(c->Vl, -1);
+      std::vector<double> wgt(c->V, 0.0);
+      for (int s = 0; s < c->Vl; ++s) wgt[c->orbit_of[s]] += 1.0;
+      for (int r = 0; r < c->V; ++r) rmap[c->rep_site[r]] = r;
+      with((void**)&c->smap_dev, c->orbit_of.data(), sizeof(int) * c->Vl);
+      with((void**)&c->rmap_dev, rmap.data(), sizeof(int) * c->Vl);
+      with((void**)&c->wgt_dev, wgt.data(), sizeof(double) * c->V);
+    }
+    with((void**)&c->m2, nullptr, 8 * sizeof(double));
+    with((void**)&c->hpart, nullptr, hartree_part_doubles(c->V) * sizeof(double));
+    with((void**)&c->flag, nullptr, 4 * sizeof(int));
+    with((void**)&c->wg0_dev, nullptr, sizeof(int));
+    with((void**)&c->st_dev, &c->st, sizeof(StepState));
+    with((void**)&c->N_dev, &c->N, sizeof(int));
+    // these two hold device addresses: filled in once the arena has one
+    const size_t stptr_off = used;
+    with((void**)&c->stptr_dev, nullptr, sizeof(StepState*));
+    const size_t margs_off = used;
+    with((void**)&c->margs_dev, nullptr, sizeof(MemintArgs));
+    if (sym || c->hstage_n == 2 * HSTAGE_MAX) place((void**)&c->modes, (size_t)6 * c->V * sizeof(double));
+    // staging: 4 lattices
+    place((void**)&c->partial, (size_t)6 * meas_groups(c->N, c->NB) * sizeof(double));
+    place((void**)&c->vbuf, 4 * (size_t)c->V * sizeof(double));
+    if ((rc = dmalloc(c, &c->arena, used))) return fail(rc);
+    for (const Part& q : parts) *q.ptr = static_cast<char*>(c->arena) + q.off;
+    c->items = c->items_r[1];
+    std::memcpy(image.data() + stptr_off, &c->st_dev, sizeof(StepState*));
+    const MemintArgs ma = memint_args(c);
+    std::memcpy(image.data() + margs_off, &ma, sizeof(MemintArgs));
+    if (hipMemcpy(c->arena, image.data(), image.size(), hipMemcpyHostToDevice) != hipSuccess) return fail(KB_ERR_HIP);
+  }
+  if (hipHostMalloc((void**)&c->hstage, (HSTAGE_SCALARS + c->hstage_n) * sizeof(double), hipHostMallocDefault) !=
+      hipSuccess)
+    return fail(KB_ERR_OOM);
+  c->hdata = c->hstage + HSTAGE_SCALARS;
   if ((rc = dmalloc(c, (void**)&c->modes, (size_t)6 * c->V * sizeof(double)))) return fail(rc);
   // staging: 4 lattices, or the 4 site-1 history vectors of kb_measure_history
   const size_t vlen = (size_t)(c->V > c->N ? c->V : c->N);
   if ((rc = dmalloc(c, (void**)&c->vbuf, 4 * vlen * sizeof(double)))) return fail(rc);
-  if ((rc = dmalloc(c, (void**)&c->tw, (size_t)p->Nx * sizeof(double2)))) return fail(rc);
-  if ((rc = dmalloc(c, (void**)&c->flag, sizeof(int) * 4))) return fail(rc);
-  // memory-integral work items: chunks of MEMINT_ROWS rows of each column
-  // block, in storage order
-  for (int i = 0; i < 3; ++i) {
-    const int rows = MEMINT_ROW_CHOICES[i];
-    std::vector<int2> items;
-    for (int J = 0; J * CB < c->N; ++J)
-      for (int k = 0; J * CB + k * rows < c->N; ++k) items.push_back(make_int2(J, k));
-    c->nitems_r[i] = (int)items.size();
-    if ((rc = dmalloc(c, (void**)&c->items_r[i], sizeof(int2) * items.size()))) return fail(rc);
-    if (hipMemcpy(c->items_r[i], items.data(), sizeof(int2) * items.size(), hipMemcpyHostToDevice) != hipSuccess)
-      return fail(KB_ERR_HIP);
-    if (rows == MEMINT_ROWS) {
-      c->items = c->items_r[i];
-      c->nitems = c->nitems_r[i];
-    }
-  }
-  if ((rc = dmalloc(c, (void**)&c->st_dev, sizeof(StepState)))) return fail(rc);
-  if ((rc = dmalloc(c, (void**)&c->stptr_dev, sizeof(StepState*)))) return fail(rc);
-  if ((rc = dmalloc(c, (void**)&c->N_dev, sizeof(int)))) return fail(rc);
-  if ((rc = dmalloc(c, (void**)&c->margs_dev, sizeof(MemintArgs)))) return fail(rc);
-  if ((rc = dmalloc(c, (void**)&c->wg0_dev, sizeof(int)))) return fail(rc);
-  {
-    const int zero = 0;
-    const MemintArgs ma = memint_args(c);
-    if (hipMemcpy(c->st_dev, &c->st, sizeof(StepState), hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(c->stptr_dev, &c->st_dev, sizeof(StepState*), hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(c->N_dev, &c->N, sizeof(int), hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(c->margs_dev, &ma, sizeof(MemintArgs), hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(c->wg0_dev, &zero, sizeof(int), hipMemcpyHostToDevice) != hipSuccess)
-      return fail(KB_ERR_HIP);
-  }
   if (sigma_planes_supported(p->Nx, p->sdim) && sigma_planes_prepare(p->Nx) != hipSuccess) {
     seterr(c, KB_ERR_ARG, "self-energy plane kernels: LDS attribute rejected");
     return fail(KB_ERR_ARG);
@@ -855,9 +985,6 @@ static int create_ctx(const kb_params* p, bool sym, kb_ctx** out) {
   if (hipMemsetAsync(c->H, 0, hcount * sizeof(double), c->stream) != hipSuccess) return fail(KB_ERR_HIP);
   if (hipMemsetAsync(c->S, 0, (size_t)c->NB * c->N * MB * 2 * sizeof(double), c->stream) != hipSuccess)
     return fail(KB_ERR_HIP);
-  if (hipMemsetAsync(c->m2, 0, 8 * sizeof(double), c->stream) != hipSuccess) return fail(KB_ERR_HIP);
-  if (hipMemsetAsync(c->hpart, 0, hartree_part_doubles(c->V) * sizeof(double), c->stream) != hipSuccess)
-    return fail(KB_ERR_HIP);
   if (c->PF) {
     for (double* ptr : {c->PF, c->PR, c->IR})
       if (hipMemsetAsync(ptr, 0, pcount * sizeof(double), c->stream) != hipSuccess) return fail(KB_ERR_HIP);
@@ -886,25 +1013,6 @@ static int create_ctx(const kb_params* p, bool sym, kb_ctx** out) {
         return fail(rc);
     }
   }
-  // twiddles exp(-2 pi i k / Nx) and the default k^2 table
-  std::vector<double2> tw(p->Nx);
-  fft_twiddles(p->Nx, tw.data());
-  std::vector<double> k2(c->Vpad, 0.0);
-  for (int i = 0; i < c->V; ++i) {
-    int rem = sym ? c->rep_site[i] : i;
-    double s2 = 0.0;
-    for (int d = 0; d < p->sdim; ++d) {
-      const int nd = rem % p->Nx;
-      rem /= p->Nx;
-      const double s = std::sin(M_PI * (double)nd / (double)p->Nx);
-      s2 += 4.0 * s * s;
-    }
-    k2[i] = s2;
-  }
-  if (hipMemcpy(c->tw, tw.data(), sizeof(double2) * p->Nx, hipMemcpyHostToDevice) != hipSuccess)
-    return fail(KB_ERR_HIP);
-  if (hipMemcpy(c->kL2, k2.data(), sizeof(double) * c->Vpad, hipMemcpyHostToDevice) != hipSuccess)
-    return fail(KB_ERR_HIP);
   if (hipStreamSynchronize(c->stream) != hipSuccess) return fail(KB_ERR_HIP);
   *out = c;
   return KB_OK;
@@ -1066,26 +1174,34 @@ int kb_measure(kb_ctx* c, int t, kb_meas* out, double* F, double* ddF, double* r
   a.dt = c->p.dt;
   a.integral = has_sigma(c);
   const bool want = F || ddF || r || n || omega || cc;
+  // the six lattices: straight into pinned host memory where they fit (orbit
+  // storage: expanded into it)
+  const bool fits = (size_t)6 * c->Vl <= c->hstage_n && c->hstage_n <= HSTAGE_MAX;
+  double* lat = fits && !c->sym ? c->hdata : c->modes;
   if (want) {
-    a.outF = c->modes;
-    a.outddF = c->modes + c->V;
-    a.outr = c->modes + 2 * c->V;
-    a.outn = c->modes + 3 * c->V;
-    a.outom = c->modes + 4 * c->V;
-    a.outc = c->modes + 5 * c->V;
+    a.outF = lat;
+    a.outddF = lat + c->V;
+    a.outr = lat + 2 * c->V;
+    a.outn = lat + 3 * c->V;
+    a.outom = lat + 4 * c->V;
+    a.outc = lat + 5 * c->V;
   }
+  a.m2 = c->m2;
+  a.workers = meas_workers(c->N);
   a.partial = c->partial;
-  const int g = meas_grid(c);
-  hipLaunchKernelGGL(measure_kernel, dim3(g), dim3(MEAS_THREADS), 0, c->stream, a);
+  a.sums = c->hstage;
+  const int groups = meas_groups(c->N, c->NB);
+  hipLaunchKernelGGL(measure_kernel, dim3(groups), dim3(MEAS_THREADS), 0, c->stream, a);
+  hipLaunchKernelGGL(measure_finish, dim3(1), dim3(MEAS_THREADS), 0, c->stream, a, groups);
   LAUNCHCHK(c);
-  std::vector<double> part((size_t)6 * g);
-  int rc;
-  if ((rc = download(c, part.data(), c->partial, part.size()))) return rc;
-  double m2 = 0;
-  if ((rc = download(c, &m2, c->m2, 1))) return rc;
-  double s[6] = {0, 0, 0, 0, 0, 0};
-  for (int b = 0; b < g; ++b)
-    for (int k = 0; k < 6; ++k) s[k] += part[(size_t)b * 6 + k];
+  if (want && fits && c->sym) {
+    hipLaunchKernelGGL(expand_kernel, dim3((c->Vl + 255) / 256), dim3(256), 0, c->stream, c->modes, c->V, c->smap_dev,
+                       c->Vl, 6, c->hdata);
+    LAUNCHCHK(c);
+  }
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  const double* s = c->hstage;
+  const double m2 = s[6];
   const double dt = c->p.dt;
   const double H = hartree_prefactor(c);
   const double ivol = 1.0 / (double)c->Vl;
@@ -1103,9 +1219,22 @@ int kb_measure(kb_ctx* c, int t, kb_meas* out, double* F, double* ddF, double* r
   out->M2 = m2;
   out->n_unstable = (int)s[5];
   double* dsts[6] = {F, ddF, r, n, omega, cc};
-  for (int k = 0; k < 6; ++k)
-    if (dsts[k] && (rc = lat_download(c, dsts[k], c->modes + (size_t)k * c->V))) return rc;
-  return KB_OK;
+  if (fits) {
+    for (int k = 0; k < 6; ++k)
+      if (dsts[k]) std::memcpy(dsts[k], c->hdata + (size_t)k * c->Vl, sizeof(double) * c->Vl);
+    return KB_OK;
+  }
+  int rc;
+  double* to[6];
+  const double* from[6];
+  int nl = 0;
+  for (int k = 0; k < 6; ++k) {
+    if (!dsts[k]) continue;
+    if (c->sym && (rc = lat_download(c, dsts[k], c->modes + (size_t)k * c->V))) return rc;
+    to[nl] = dsts[k];
+    from[nl++] = c->modes + (size_t)k * c->V;
+  }
+  return c->sym || !nl ? KB_OK : download_many(c, nl, to, from, c->V);
 }
 
 int kb_measure_history(kb_ctx* c, int t, double* SigF, double* Sigr, double* Fonet, double* ronet) {
@@ -1114,14 +1243,12 @@ int kb_measure_history(kb_ctx* c, int t, double* SigF, double* Sigr, double* Fon
   const int L = t - c->st.tmin;
   if (L <= 0) return KB_OK;
   hipLaunchKernelGGL(history_kernel, dim3((L + 255) / 256), dim3(256), 0, c->stream, c->H, c->S, c->NP, c->N,
-                     c->st.tmin, t, c->vbuf);
+                     c->st.tmin, t, c->hdata);  // 4 L values: hstage_n >= 4 N
   LAUNCHCHK(c);
-  std::vector<double> h((size_t)4 * L);
-  int rc;
-  if ((rc = download(c, h.data(), c->vbuf, h.size()))) return rc;
+  HIPCHK(c, hipStreamSynchronize(c->stream));
   double* dsts[4] = {SigF, Sigr, Fonet, ronet};
   for (int k = 0; k < 4; ++k)
-    if (dsts[k]) memcpy(dsts[k], h.data() + (size_t)k * L, sizeof(double) * L);
+    if (dsts[k]) memcpy(dsts[k], c->hdata + (size_t)k * L, sizeof(double) * L);
   return KB_OK;
 }
 
@@ -1131,10 +1258,11 @@ int kb_get_entry(kb_ctx* c, int which, int i, int j, double* out) {
     return seterr(c, KB_ERR_WINDOW, "get: (%d,%d) outside window [%d,%d]", i, j, c->st.tmin, c->st.tmax);
   const int si = slot_of(c, i), sj = slot_of(c, j);
   const double sg = which ? (si >= sj ? 1.0 : -1.0) : 1.0;
+  double* o = lattice_out(c);
   hipLaunchKernelGGL(gather_pair, dim3((c->V + 255) / 256), dim3(256), 0, c->stream, c->H, c->NP, c->V,
-                     pair_off(si, sj, c->N), which, sg, c->vbuf);
+                     pair_off(si, sj, c->N), which, sg, o);
   LAUNCHCHK(c);
-  return lat_download(c, out, c->vbuf);
+  return deliver(c, out, o);
 }
 
 int kb_set_entry(kb_ctx* c, int which, int i, int j, const double* in) {
@@ -1156,10 +1284,11 @@ int kb_set_entry(kb_ctx* c, int which, int i, int j, const double* in) {
 int kb_get_sigma(kb_ctx* c, int which, int tp, double* out) {
   if (!c || !out || (which != 0 && which != 1)) return KB_ERR_ARG;
   if (!inwin(c, tp)) return seterr(c, KB_ERR_WINDOW, "sigma: %d outside window [%d,%d]", tp, c->st.tmin, c->st.tmax);
+  double* o = lattice_out(c);
   hipLaunchKernelGGL(gather_sigma, dim3((c->V + 255) / 256), dim3(256), 0, c->stream, c->S, c->N, c->V,
-                     slot_of(c, tp), which, c->vbuf);
+                     slot_of(c, tp), which, o);
   LAUNCHCHK(c);
-  return lat_download(c, out, c->vbuf);
+  return deliver(c, out, o);
 }
 
 int kb_read_bandwidth(int device, long long bytes, double* gbs) {
@@ -1195,12 +1324,13 @@ int kb_read_bandwidth(int device, long long bytes, double* gbs) {
 int kb_ninv_get(kb_ctx* c, int which, int i, int j, double* out) {
   if (!c || !out || which < 0 || which > 4) return KB_ERR_ARG;
   if (c->p.pexp != KB_PEXP_NINVERSE_NLO) return seterr(c, KB_ERR_STATE, "no 1/N resummation in this context");
+  double* o = lattice_out(c);
   if (which >= 3) {
     if (!inwin(c, j) || c->st.tmax < 3) return seterr(c, KB_ERR_WINDOW, "ring: %d outside window [%d,%d]", j, c->st.tmin, c->st.tmax);
     hipLaunchKernelGGL(gather_sigma, dim3((c->V + 255) / 256), dim3(256), 0, c->stream, c->Iring, c->N, c->V,
-                       slot_of(c, j), which == 3 ? 0 : 1, c->vbuf);
+                       slot_of(c, j), which == 3 ? 0 : 1, o);
     LAUNCHCHK(c);
-    return lat_download(c, out, c->vbuf);
+    return deliver(c, out, o);
   }
   if (!inwin(c, i) || !inwin(c, j) || (which == 2 && i <= j))
     return seterr(c, KB_ERR_WINDOW, "1/N entry (%d,%d) outside window [%d,%d]", i, j, c->st.tmin, c->st.tmax);
@@ -1208,9 +1338,9 @@ int kb_ninv_get(kb_ctx* c, int which, int i, int j, double* out) {
   const double* src = which == 0 ? c->PF : which == 1 ? c->PR : c->IR;
   const double sg = which == 1 ? (si >= sj ? 1.0 : -1.0) : 1.0;
   hipLaunchKernelGGL(gather_tri, dim3((c->V + 255) / 256), dim3(256), 0, c->stream, src, c->PNP, c->V,
-                     ppair_off(si, sj, c->N), sg, c->vbuf);
+                     ppair_off(si, sj, c->N), sg, o);
   LAUNCHCHK(c);
-  return lat_download(c, out, c->vbuf);
+  return deliver(c, out, o);
 }
 
 int kb_check_finite(kb_ctx* c) {

@@ -24,6 +24,9 @@ struct EventPair {
 // 5 the 1/N resummation sweeps
 constexpr int NSTAGE = 6;
 
+constexpr size_t HSTAGE_SCALARS = 16;           // doubles before the lattices
+constexpr size_t HSTAGE_MAX = size_t(1) << 20;  // doubles: 8 MiB
+
 struct AdjState;  // kb_adjoint.hip
 
 }  // namespace qftkb_host
@@ -48,7 +51,9 @@ struct kb_ctx {
   bool in_ensemble = false;
   double initmass = 0.0;      // set by kb_init_particles
   bool init_particles = false;
-  // device memory
+  // device memory; the small buffers (from m2 on, the maps above and the
+  // launch tables below) share one allocation
+  void* arena = nullptr;
   double* H = nullptr;     // history
   double* S = nullptr;     // self-energy ring
   double2* W = nullptr;    // FFT workspace
@@ -58,6 +63,12 @@ struct kb_ctx {
   double* partial = nullptr;
   double* modes = nullptr; // 6 x V measurement outputs
   double* vbuf = nullptr;  // 4 x V staging
+  // pinned host memory through which results leave the device: the scalars
+  // of a measurement, then hstage_n doubles of lattices (all six of a
+  // measurement where they fit HSTAGE_MAX, else two buffers of half that)
+  double* hstage = nullptr;
+  double* hdata = nullptr;
+  size_t hstage_n = 0;
   double2* tw = nullptr;
   int* flag = nullptr;
   int2* items = nullptr;  // memory-integral work items of 64-row chunks (adjoint kernels, ensembles)

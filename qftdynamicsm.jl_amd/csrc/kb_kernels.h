@@ -181,7 +181,10 @@ struct MeasArgs {
   double dt;
   int integral;
   double *outF, *outddF, *outr, *outn, *outom, *outc;
-  double* partial;
+  const double* m2;
+  int workers;      // meas_workers(N)
+  double* partial;  // 6 sums per workgroup
+  double* sums;     // the 6 sums over all sites, and *m2
 };
 
 __global__ void sigma_pass(SigmaArgs a);
@@ -233,6 +236,8 @@ extern const MemintVariant kMemintVariants[NMEMINT_VARIANTS];
 constexpr int MEMINT_ROW_CHOICES[3] = {32, 64, 128};  // item tables kept per context
 __global__ void advance_kernel(StepState* const* states, const int* Ns, int nruns);
 __global__ void measure_kernel(MeasArgs a);
+__global__ void measure_finish(MeasArgs a, int groups);
+__global__ void expand_kernel(const double* src, int V, const int* smap, int Vl, int narr, double* dst);
 __global__ void history_kernel(const double* H, const double* S, long NP, int N, int tmin, int t, double* out);
 __global__ void gather_pair(const double* H, long NP, int V, long pair, int comp, double sign, double* out);
 __global__ void scatter_pair(double* H, long NP, int V, long pair, int comp, double sign, const double* in);
@@ -303,6 +308,19 @@ constexpr int MEMINT_THREADS = 256;  // default workgroup of the memory-integral
 constexpr int MEMINT_FINISH_THREADS = 1024;
 constexpr int MEMINT_ROWS = 64;  // rows per work item of the adjoint kernels
 constexpr int MEAS_THREADS = 256;
+// 8-lane workers that share the times of a site block in measure_kernel, a
+// power of two: about four times each, one round of its loads in flight
+inline int meas_workers(int N) {
+  int w = 1;
+  while (w < MEAS_THREADS / MB && 4 * w < N) w *= 2;
+  return w;
+}
+constexpr int MEAS_GROUPS = 1024;
+inline int meas_groups(int N, int NB) {
+  const int per = MEAS_THREADS / MB / meas_workers(N);
+  const int g = (NB + per - 1) / per;
+  return g < MEAS_GROUPS ? g : MEAS_GROUPS;
+}
 
 }  // namespace qftkb
 

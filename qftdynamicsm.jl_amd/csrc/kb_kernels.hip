@@ -1078,69 +1078,126 @@ const MemintVariant kMemintVariants[NMEMINT_VARIANTS] = {
 
 // ---------------------------------------------------------------------------
 // Measurement (createMeasurement / getE_kin / getE_pot / getE_mem)
-// partial sums per workgroup: [0] sum ddF/2, [1] sum F, [2] sum kL2 F,
-// [3] E_mem boundary integrand, [4] E_mem interior integrand, [5] n_unstable
+// sums over the sites: [0] ddF/2, [1] F, [2] kL2 F, [3] E_mem boundary
+// integrand, [4] E_mem interior integrand, [5] n_unstable
+// The E_mem integrand walks row t-1 of the history, one line per time, so one
+// thread per site was a chain of N_mem dependent rounds (252 us at 32^3,
+// N_mem = 400, on 128 workgroups).  meas_workers(N) 8-lane workers share a
+// site block's times instead, four times in flight each, on up to
+// MEAS_GROUPS workgroups; measure_finish adds their sums in workgroup order
+// into host memory.  (A last-workgroup counter instead of the second kernel
+// costs some 35 ns per workgroup: 75 us with 2048 of them.)
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void measure_kernel(MeasArgs a) {
-  __shared__ double red[6][256];
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(MEAS_THREADS) void measure_kernel(MeasArgs a) {
+  __shared__ double red[MEAS_THREADS / 64][6];
+  const int tid = threadIdx.x, lane = tid & (MB - 1), worker = tid >> 3;
+  const int wpb = a.workers;
+  const int w = worker & (wpb - 1);
+  const int per = MEAS_THREADS / MB / wpb;  // site blocks per round
   double v[6] = {0, 0, 0, 0, 0, 0};
-  if (p < a.V) {
-    const int mb = p / MB, lane = p % MB;
+  for (int mb = blockIdx.x * per + worker / wpb; mb * MB + lane < a.V; mb += gridDim.x * per) {
+    const int p = mb * MB + lane;
     const double dt = a.dt;
-    const double Ftt = a.H[hoff(mb, pair_off(a.s_t, a.s_t, a.N), lane, a.NP)];
-    const double Fmt = a.H[hoff(mb, pair_off(a.s_tm1, a.s_t, a.N), lane, a.NP)];
-    const double* emm = a.H + hoff(mb, pair_off(a.s_tm1, a.s_tm1, a.N), lane, a.NP);
-    const double Fmm = emm[0];
-    const double ddF = (Ftt - 2.0 * Fmt + Fmm) / (dt * dt);
-    const double om = (ddF / Fmm) > 0 ? sqrt(ddF / Fmm) : 0.0;
-    double c;
-    int bad = 0;
-    if (0.25 * (dt * dt) * (om * om) < 1.0) {
-      c = sqrt(1.0 - 0.25 * (dt * dt) * (om * om));
-    } else {
-      c = 1.0;
-      bad = 1;
-    }
-    const double nn = (ddF * Fmm > 0) ? (c * sqrt(ddF * Fmm)) - 0.5 : 0.0;
-    if (a.outF) {
-      a.outF[p] = Fmm;
-      a.outddF[p] = ddF;
-      a.outr[p] = emm[1];
-      a.outn[p] = nn;
-      a.outom[p] = om;
-      a.outc[p] = c;
-    }
+    const double* Hb = a.H + hoff(mb, 0, lane, a.NP);
     const double g = a.wgt ? a.wgt[p] : 1.0;
-    v[0] = g * 0.5 * ddF;
-    v[1] = g * Fmm;
-    v[2] = g * a.kL2[p] * Fmm;
-    v[5] = g * bad;
+    if (w == 0) {
+      const double Ftt = Hb[pair_rel(a.s_t, a.s_t, a.N)];
+      const double Fmt = Hb[pair_rel(a.s_tm1, a.s_t, a.N)];
+      const double2 emm = ld_global(Hb + pair_rel(a.s_tm1, a.s_tm1, a.N));
+      const double Fmm = emm.x;
+      const double ddF = (Ftt - 2.0 * Fmt + Fmm) / (dt * dt);
+      const double om = (ddF / Fmm) > 0 ? sqrt(ddF / Fmm) : 0.0;
+      double c;
+      int bad = 0;
+      if (0.25 * (dt * dt) * (om * om) < 1.0) {
+        c = sqrt(1.0 - 0.25 * (dt * dt) * (om * om));
+      } else {
+        c = 1.0;
+        bad = 1;
+      }
+      const double nn = (ddF * Fmm > 0) ? (c * sqrt(ddF * Fmm)) - 0.5 : 0.0;
+      if (a.outF) {
+        a.outF[p] = Fmm;
+        a.outddF[p] = ddF;
+        a.outr[p] = emm.y;
+        a.outn[p] = nn;
+        a.outom[p] = om;
+        a.outc[p] = c;
+      }
+      v[0] += g * 0.5 * ddF;
+      v[1] += g * Fmm;
+      v[2] += g * a.kL2[p] * Fmm;
+      v[5] += g * bad;
+    }
     if (a.t != 2 && a.integral) {
       // E_mem integrand over t' in [tmin, t-2] against F(t',t-1), rho(t',t-1)
-      for (int tp = a.tmin; tp <= a.t - 2; ++tp) {
-        const int x = (tp - 1) % a.N;
-        const double* e = a.H + hoff(mb, pair_off(x, a.s_tm1, a.N), lane, a.NP);
-        const double rr = e[1] * (x >= a.s_tm1 ? 1.0 : -1.0);
-        const double* S = a.S + soff(mb, x, lane, a.N);
-        const double term = g * (S[1] * e[0] - S[0] * rr);
-        if (tp == a.tmin)
-          v[3] += term;
-        else
-          v[4] += term;
+      const int smin = (a.tmin - 1) % a.N;
+      const int n = a.t - 1 - a.tmin;
+      const double* Sb = a.S + soff(mb, 0, lane, a.N);
+      constexpr int U = 4;
+      for (int q0 = w; q0 < n; q0 += wpb * U) {
+        double2 e[U], sg[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int q = min(q0 + u * wpb, n - 1);
+          const int x = smin + q < a.N ? smin + q : smin + q - a.N;
+          e[u] = ld_global(Hb + pair_rel(x, a.s_tm1, a.N));
+          sg[u] = ld_global(Sb + x * (2 * MB));
+          if (x < a.s_tm1) e[u].y = -e[u].y;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int q = q0 + u * wpb;
+          const double term = g * (sg[u].y * e[u].x - sg[u].x * e[u].y);
+          if (q == 0)
+            v[3] += term;
+          else if (q < n)
+            v[4] += term;
+        }
       }
     }
   }
 #pragma unroll
-  for (int k = 0; k < 6; ++k) red[k][threadIdx.x] = v[k];
+  for (int k = 0; k < 6; ++k)
+    for (int o = 32; o > 0; o >>= 1) v[k] += __shfl_xor(v[k], o);
+  if ((tid & 63) == 0)
+    for (int k = 0; k < 6; ++k) red[tid >> 6][k] = v[k];
   __syncthreads();
-  for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w)
-#pragma unroll
-      for (int k = 0; k < 6; ++k) red[k][threadIdx.x] += red[k][threadIdx.x + w];
-    __syncthreads();
+  if (tid < 6) {
+    double t = 0.0;
+    for (int q = 0; q < MEAS_THREADS / 64; ++q) t += red[q][tid];
+    a.partial[(size_t)blockIdx.x * 6 + tid] = t;
   }
-  if (threadIdx.x < 6) a.partial[blockIdx.x * 6 + threadIdx.x] = red[threadIdx.x][0];
+}
+
+__global__ __launch_bounds__(MEAS_THREADS) void measure_finish(MeasArgs a, int G) {
+  __shared__ double red[MEAS_THREADS / 64][6];
+  const int tid = threadIdx.x;
+  double v[6] = {0, 0, 0, 0, 0, 0};
+  for (int b = tid; b < G; b += MEAS_THREADS)
+#pragma unroll
+    for (int k = 0; k < 6; ++k) v[k] += a.partial[(size_t)b * 6 + k];
+#pragma unroll
+  for (int k = 0; k < 6; ++k)
+    for (int o = 32; o > 0; o >>= 1) v[k] += __shfl_xor(v[k], o);
+  if ((tid & 63) == 0)
+    for (int k = 0; k < 6; ++k) red[tid >> 6][k] = v[k];
+  __syncthreads();
+  if (tid < 6) {
+    double t = 0.0;
+    for (int q = 0; q < MEAS_THREADS / 64; ++q) t += red[q][tid];
+    a.sums[tid] = t;
+  }
+  if (tid == 6) a.sums[6] = a.m2[0];
+}
+
+// narr arrays of V stored sites to the whole lattice (orbit storage)
+__global__ void expand_kernel(const double* __restrict__ src, int V, const int* __restrict__ smap, int Vl, int narr,
+                              double* __restrict__ dst) {
+  const int s = blockIdx.x * blockDim.x + threadIdx.x;
+  if (s >= Vl) return;
+  const int r = smap[s];
+  for (int k = 0; k < narr; ++k) dst[(size_t)k * Vl + s] = src[(size_t)k * V + r];
 }
 
 // site-1 history (Measurement.jl:90-96); q = 0 .. t-tmin-1
