@@ -234,8 +234,9 @@ int kb_tile_shape(int variant, int *rows, int *batch, int *threads); /* KB_ERR_A
 int kb_set_tiles(kb_ctx *ctx, int variant);
 int kb_get_tiles(const kb_ctx *ctx, int *variant);
 int kb_autotune(kb_ctx *ctx, int reps, int *best, double *ms);
-/* The same for the self-energy stage's plane kernels (threads per
- * workgroup); re-running the stage recomputes the same self-energies.
+/* The same for the self-energy stage's transforms (threads per
+ * workgroup asked for; sizes whose passes are compiled for their length have
+ * their own); re-running the stage recomputes the same self-energies.
  * Orbit-storage LambdaNLO and NinverseNLO contexts (kb_create_sym, up to
  * 4096 orbits) have one more form, KB_FFT_ORBIT_PRODUCT, their default: the
  * transforms of the sunset (or of the 1/N bubble and chain passes) as FP64

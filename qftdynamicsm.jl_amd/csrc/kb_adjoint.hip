@@ -975,10 +975,7 @@ int launch_sigma_adjoint(kb_ctx* c) {
   a.Sbar = s->Sbar;
   a.Hbar = s->Hbar;
   a.classical = c->p.pexp == KB_PEXP_LAMBDA_NLO_CLASSICAL;
-  a.P = c->fftP;
-  a.npencils = c->V / c->p.Nx;
-  hipError_t e = sigma_planes_supported(c->p.Nx, c->p.sdim) ? launch_sigma_planes_adjoint(a, c->N - 1, c->stream)
-                                                            : launch_sunset_adjoint_pencils(a, c->N - 1, c->stream);
+  hipError_t e = launch_sigma_stage(a, SG_SUNSET_ADJ, c->N - 1, c->stream);
   if (e != hipSuccess) return seterr(c, KB_ERR_HIP, "adjoint self-energy launch failed: %s", hipGetErrorString(e));
   return KB_OK;
 }

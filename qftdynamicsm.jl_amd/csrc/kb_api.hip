@@ -54,16 +54,6 @@ int seterr(kb_ctx* c, int code, const char* fmt, ...) {
 inline int slot_of(const kb_ctx* c, int t) { return (t - 1) % c->N; }
 inline bool inwin(const kb_ctx* c, int t) { return c->st.tmin <= t && t <= c->st.tmax; }
 
-void plan_fft(FFTPlan& pl, int n) {
-  pl.n = n;
-  pl.nf = 0;
-  int m = n;
-  while (m % 4 == 0 && pl.nf < FFT_MAXF) { pl.fac[pl.nf++] = 4; m /= 4; }
-  while (m % 2 == 0 && pl.nf < FFT_MAXF) { pl.fac[pl.nf++] = 2; m /= 2; }
-  for (int f = 3; m > 1 && pl.nf < FFT_MAXF; f += 2)
-    while (m % f == 0) { pl.fac[pl.nf++] = f; m /= f; }
-}
-
 void fft_twiddles(int n, double2* out) {
   for (int k = 0; k < n; ++k) {
     long double a = -2.0L * 3.14159265358979323846264338327950288L * (long double)k / (long double)n;
@@ -189,8 +179,6 @@ int launch_sigma(kb_ctx* c, double2* X, double* S_out) {
   a.nx = c->nx;
   a.ny = c->ny;
   a.nz = c->nz;
-  a.P = c->fftP;
-  a.npencils = c->Vl / c->p.Nx;
   a.st = c->st_dev;
   a.preF = ivol * ivol * ivol * (-(lam * lam) * (ON + 2.0) / (18.0 * ON * ON));
   a.preR = ivol * ivol * ivol * (-(lam * lam) * (ON + 2.0) / (6.0 * ON * ON));
@@ -205,41 +193,8 @@ int launch_sigma(kb_ctx* c, double2* X, double* S_out) {
     return KB_OK;
   }
   if (plane_workspace_missing(c)) return seterr(c, KB_ERR_STATE, "self-energy: plane workspace not allocated");
-  if (sigma_planes_supported(c->p.Nx, c->p.sdim)) {
-    hipError_t e = launch_sigma_planes(a, L, c->stream, c->fft_tile);
-    if (e != hipSuccess) return seterr(c, KB_ERR_HIP, "self-energy launch failed: %s", hipGetErrorString(e));
-    return KB_OK;
-  }
-  if (X) {
-    // the adjoint's recompute keeps the forward transforms: the pencil passes
-    // that save them (2D and 3D past the plane kernels)
-    hipError_t e = launch_sunset_pencils(a, L, c->stream);
-    if (e != hipSuccess) return seterr(c, KB_ERR_HIP, "self-energy launch failed: %s", hipGetErrorString(e));
-    return KB_OK;
-  }
-  const size_t lds = sizeof(double2) * 2 * (size_t)a.P * a.n;
-  const dim3 grid((a.npencils + a.P - 1) / a.P, L);
-  std::vector<std::pair<int, int>> passes;  // (axis, flags)
-  const int sd = c->p.sdim;
-  if (sd == 1) {
-    passes.push_back({0, SIGMA_GATHER | SIGMA_SUNSET | SIGMA_SCATTER});
-  } else if (sd == 2) {
-    passes.push_back({0, SIGMA_GATHER});
-    passes.push_back({1, SIGMA_SUNSET});
-    passes.push_back({0, SIGMA_INVERSE | SIGMA_SCATTER});
-  } else {
-    passes.push_back({0, SIGMA_GATHER});
-    passes.push_back({1, 0});
-    passes.push_back({2, SIGMA_SUNSET});
-    passes.push_back({1, SIGMA_INVERSE});
-    passes.push_back({0, SIGMA_INVERSE | SIGMA_SCATTER});
-  }
-  for (auto& ps : passes) {
-    a.axis = ps.first;
-    a.flags = ps.second;
-    hipLaunchKernelGGL(sigma_pass, grid, dim3(256), lds, c->stream, a);
-    LAUNCHCHK(c);
-  }
+  hipError_t e = launch_sigma_stage(a, SG_SUNSET, L, c->stream, c->fft_tile);
+  if (e != hipSuccess) return seterr(c, KB_ERR_HIP, "self-energy launch failed: %s", hipGetErrorString(e));
   return KB_OK;
 }
 
@@ -263,8 +218,6 @@ SigmaArgs ninv_sigma_args(kb_ctx* c, const StepState* st) {
   a.nx = c->nx;
   a.ny = c->ny;
   a.nz = c->nz;
-  a.P = c->fftP;
-  a.npencils = c->Vl / c->p.Nx;
   a.st = st;
   a.PF = c->PF;
   a.PR = c->PR;
@@ -289,8 +242,7 @@ int launch_bubble(kb_ctx* c, const StepState* st, bool keep) {
   SigmaArgs a = ninv_sigma_args(c, st);
   a.preF = a.preR = ivol * ivol;
   a.X = keep ? c->Xn : nullptr;
-  hipError_t e = sigma_planes_supported(c->p.Nx, c->p.sdim) ? launch_bubble_planes(a, c->N - 1, c->stream)
-                                                            : launch_bubble_pencils(a, c->N - 1, c->stream);
+  hipError_t e = launch_sigma_stage(a, SG_BUBBLE, c->N - 1, c->stream);
   if (e != hipSuccess) return seterr(c, KB_ERR_HIP, "bubble launch failed: %s", hipGetErrorString(e));
   return KB_OK;
 }
@@ -344,8 +296,7 @@ int launch_chain(kb_ctx* c) {
   SigmaArgs a = ninv_sigma_args(c, c->st_dev);
   a.preF = a.preR = pre;
   a.X = c->Xn;
-  hipError_t e = sigma_planes_supported(c->p.Nx, c->p.sdim) ? launch_chain_planes(a, c->N - 1, c->stream)
-                                                            : launch_chain_pencils(a, c->N - 1, c->stream);
+  hipError_t e = launch_sigma_stage(a, SG_CHAIN, c->N - 1, c->stream);
   if (e != hipSuccess) return seterr(c, KB_ERR_HIP, "chain launch failed: %s", hipGetErrorString(e));
   return KB_OK;
 }
@@ -640,29 +591,23 @@ int dmalloc(kb_ctx* c, void** ptr, size_t bytes) {
   return KB_OK;
 }
 
-// The plane kernels' workspace: W holds one complex lattice per row between
-// the passes (3D lattices, and the pencil passes past Nx = 64); Xn keeps the
-// 1/N bubble pass's transforms for its chain pass.  Allocated when a plane
-// form is first selected: LambdaLO and contexts on the orbit products never
-// hold them.
+// The transform passes' workspace: W holds the half space of each row between
+// the passes; Xn keeps the 1/N bubble pass's transforms for its chain pass.
+// Allocated when that form of the stage is first selected: LambdaLO and
+// contexts on the orbit products never hold them.
 int ensure_plane_workspace(kb_ctx* c) {
   if (!has_sigma(c)) return KB_OK;
   int rc;
   const size_t rows = (size_t)c->N * c->Vl * sizeof(double2);
-  // the plane passes keep the half space z in [0, Nx/2] of each row; the
-  // pencil passes (Nx > 64) whole rows
-  const int n = c->p.Nx;
-  const size_t wrows = sigma_planes_supported(n, c->p.sdim) ? (size_t)c->N * n * n * (n / 2 + 1) * sizeof(double2) : rows;
-  if ((c->p.sdim == 3 || !sigma_planes_supported(n, c->p.sdim)) && !c->W && (rc = dmalloc(c, (void**)&c->W, wrows)))
-    return rc;
+  const size_t wvals = sigma_workspace_values(c->p.Nx, c->p.sdim, c->N);
+  if (wvals && !c->W && (rc = dmalloc(c, (void**)&c->W, wvals * sizeof(double2)))) return rc;
   if (c->p.pexp == KB_PEXP_NINVERSE_NLO && !c->Xn && (rc = dmalloc(c, (void**)&c->Xn, rows))) return rc;
   return KB_OK;
 }
 
 // a plane-kernel stage needs its workspace (a guard, not a path callers reach)
 bool plane_workspace_missing(const kb_ctx* c) {
-  return ((c->p.sdim == 3 || !sigma_planes_supported(c->p.Nx, c->p.sdim)) && !c->W) ||
-         (c->p.pexp == KB_PEXP_NINVERSE_NLO && !c->Xn);
+  return (sigma_workspace_values(c->p.Nx, c->p.sdim, 1) && !c->W) || (c->p.pexp == KB_PEXP_NINVERSE_NLO && !c->Xn);
 }
 
 void cubic_orbits(int Nx, int sdim, std::vector<int>& orbit_of, std::vector<int>& rep_site) {
@@ -764,11 +709,6 @@ static int create_ctx(const kb_params* p, bool sym, kb_ctx** out) {
   c->NB = (c->V + MB - 1) / MB;
   c->Vpad = c->NB * MB;
   plan_fft(c->plan, p->Nx);
-  // pencils per workgroup: 16 complex elements per pencil row at least, and
-  // the two LDS buffers (2 P Nx complex values) within 64 KiB
-  c->fftP = p->Nx >= 64 ? 4 : (p->Nx >= 16 ? 16 : 32);
-  c->fftP = std::min(c->fftP, std::max(1, KB_MAX_NX / p->Nx));
-  if (c->fftP > c->Vl / p->Nx) c->fftP = c->Vl / p->Nx;
   int rc;
   auto fail = [&](int code) {
     free_all(c);
@@ -939,8 +879,8 @@ static int create_ctx(const kb_params* p, bool sym, kb_ctx** out) {
   // staging: 4 lattices, or the 4 site-1 history vectors of kb_measure_history
   const size_t vlen = (size_t)(c->V > c->N ? c->V : c->N);
   if ((rc = dmalloc(c, (void**)&c->vbuf, 4 * vlen * sizeof(double)))) return fail(rc);
-  if (sigma_planes_supported(p->Nx, p->sdim) && sigma_planes_prepare(p->Nx) != hipSuccess) {
-    seterr(c, KB_ERR_ARG, "self-energy plane kernels: LDS attribute rejected");
+  if (sigma_prepare() != hipSuccess) {
+    seterr(c, KB_ERR_ARG, "self-energy passes: LDS attribute rejected");
     return fail(KB_ERR_ARG);
   }
   {

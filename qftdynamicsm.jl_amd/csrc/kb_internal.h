@@ -101,7 +101,6 @@ struct kb_ctx {
   hipGraphExec_t gexec = nullptr;
   size_t bytes = 0;
   qftkb::FFTPlan plan{};
-  int fftP = 1;
   hipStream_t own = nullptr;
   hipStream_t stream = nullptr;
   bool timing = false;
@@ -146,9 +145,8 @@ struct kb_ctx {
 namespace qftkb_host {
 
 int seterr(kb_ctx* c, int code, const char* fmt, ...);
-// FFT factorisation and the twiddles exp(-2 pi i k / n), k < n (long double
-// on the host), shared by contexts and the context-free entry points
-void plan_fft(qftkb::FFTPlan& pl, int n);
+// the twiddles exp(-2 pi i k / n), k < n (long double on the host), shared by
+// contexts and the context-free entry points
 void fft_twiddles(int n, double2* out);
 // message of the calling thread's last failed context-free call
 const char* free_call_error();

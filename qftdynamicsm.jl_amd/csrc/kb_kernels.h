@@ -17,13 +17,6 @@ struct FFTPlan {
   int fac[FFT_MAXF];
 };
 
-enum SigmaFlags {
-  SIGMA_GATHER = 1,   // read F(t-1,t'), rho(t-1,t') from the history (axis 0, forward)
-  SIGMA_SUNSET = 2,   // after the forward transform: pointwise sunset, inverse transform
-  SIGMA_SCATTER = 4,  // write SigF/Sigr to the self-energy ring (axis 0, inverse)
-  SIGMA_INVERSE = 8,  // transform direction of a plain pass
-};
-
 // Window of the step being taken, after expandSimData! (SimDataStruct.jl:
 // 262-278).  Kept in device memory and advanced by advance_kernel, so a
 // step's kernels have step-invariant arguments and can be replayed from a
@@ -83,12 +76,11 @@ enum SigmaMode { SG_SUNSET = 0, SG_SUNSET_ADJ = 1, SG_BUBBLE = 2, SG_CHAIN = 3, 
 struct SigmaArgs {
   const double* H;
   double* S;
-  double2* W;  // workspace rows [N-1][V] complex
+  double2* W;  // half-space workspace rows (sigma_workspace_values)
   const double2* tw;
   FFTPlan plan;
   long NP;
   int N, V, n, nx, ny, nz;
-  int axis, flags, P, npencils;
   const StepState* st;  // rows q < st->L (t' = tmin + q) are live
   double preF, preR;
   double2* X;           // forward: if set, receives (Fx, rx) per row and site; adjoint: read
@@ -187,7 +179,6 @@ struct MeasArgs {
   double* sums;     // the 6 sums over all sites, and *m2
 };
 
-__global__ void sigma_pass(SigmaArgs a);
 // wgt: sites each stored site stands for (orbit storage), NULL = 1
 __global__ void hartree_kernel(const double* H, long NP, int V, long pair, double hfac, double Mass2,
                                const double* wgt, double* out);
@@ -252,26 +243,20 @@ __global__ void fill_free_kernel(double* H, long NP, int V, int N, int tmax, con
                                  double mass, double dt, int nb);
 __global__ void finite_kernel(const double* H, size_t count, int* flag);
 
-// self-energy stage on whole planes (kb_sigma.hip), Nx <= 64
-// the plane kernels take Nx <= 64, and 1D rows up to 2048 points (one line in LDS)
+// self-energy stage by lattice transforms (kb_sigma.hip)
+// factors of a transform length, in stage order
+void plan_fft(FFTPlan& pl, int n);
+// complex values of the workspace for `rows` rows: the half space of each
+// row, 0 where a row is transformed in one pass (1D, 2D up to a plane per
+// workgroup)
+size_t sigma_workspace_values(int Nx, int sdim, size_t rows);
+// the sizes whose stage serves orbit storage: Nx <= 64, and 1D up to 2048
 bool sigma_planes_supported(int Nx, int sdim);
-hipError_t sigma_planes_prepare(int n);
-// variant: index into kFFTThreads (threads per workgroup of the plane kernels)
+hipError_t sigma_prepare();  // LDS attribute of the passes
+// variant: index into kFFTThreads (threads per workgroup asked for)
 constexpr int NFFT_VARIANTS = 4;
 extern const int kFFTThreads[NFFT_VARIANTS];
-hipError_t launch_sigma_planes(const SigmaArgs& a, int rows, hipStream_t st, int variant = 0);
-hipError_t launch_sigma_planes_adjoint(const SigmaArgs& a, int rows, hipStream_t st);
-// the sunset of a.rows caller lattices (SG_PLAIN), default block size
-hipError_t launch_sigma_planes_plain(const SigmaArgs& a, hipStream_t st);
-hipError_t launch_bubble_planes(const SigmaArgs& a, int rows, hipStream_t st);
-hipError_t launch_chain_planes(const SigmaArgs& a, int rows, hipStream_t st);
-// the same passes on 2D and 3D lattices past the plane kernels (pencils of
-// whole rows in W)
-hipError_t launch_bubble_pencils(const SigmaArgs& a, int rows, hipStream_t st);
-hipError_t launch_chain_pencils(const SigmaArgs& a, int rows, hipStream_t st);
-// the sunset keeping its transforms in a.X, and its adjoint, as pencil passes
-hipError_t launch_sunset_pencils(const SigmaArgs& a, int rows, hipStream_t st);
-hipError_t launch_sunset_adjoint_pencils(const SigmaArgs& a, int rows, hipStream_t st);
+hipError_t launch_sigma_stage(const SigmaArgs& a, SigmaMode mode, int rows, hipStream_t st, int variant = 0);
 
 // self-energy stage of a cubic-orbit-stored window as two FP64 matrix
 // products with the orbit cosine matrix Mo (kb_orbit.hip)

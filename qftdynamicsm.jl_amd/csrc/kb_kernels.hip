@@ -1,8 +1,5 @@
 // kb_kernels.hip -- gfx950 kernels of the 2PI Kadanoff-Baym step.
 //
-//   sigma_pass     self-energy: batched pencil FFTs staged in LDS with the
-//                  sunset products fused into the last forward pass
-//                  (TwoPIScalar_Evolution.jl:16-31)
 //   hartree        Hartree mass^2 reduction (TwoPIScalar_Initialization.jl:
 //                  207-218)
 //   memint_step    memory integrals + leapfrog + diagonal of one KB step,
@@ -17,235 +14,6 @@
 #include <math.h>
 
 namespace qftkb {
-
-// ---------------------------------------------------------------------------
-// LDS FFT (Stockham, mixed radix)
-// ---------------------------------------------------------------------------
-__device__ inline double2 cmul(double2 a, double2 b) {
-  return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
-}
-__device__ inline double2 cadd(double2 a, double2 b) { return make_double2(a.x + b.x, a.y + b.y); }
-__device__ inline double2 csub(double2 a, double2 b) { return make_double2(a.x - b.x, a.y - b.y); }
-
-// exp(-+ 2 pi i k / n) from the table, conjugated for the inverse
-__device__ inline double2 twid(const double2* __restrict__ tw, int k, bool inv) {
-  double2 w = tw[k];
-  if (inv) w.y = -w.y;
-  return w;
-}
-
-template <int R>
-__device__ inline void small_dft(double2 (&v)[R], const double2* __restrict__ tw, int n, bool inv) {
-  if constexpr (R == 2) {
-    double2 a = v[0], b = v[1];
-    v[0] = cadd(a, b);
-    v[1] = csub(a, b);
-  } else if constexpr (R == 4) {
-    // forward: multiply by -i for the odd quarter; inverse: +i
-    double2 a0 = cadd(v[0], v[2]), a1 = csub(v[0], v[2]);
-    double2 b0 = cadd(v[1], v[3]), b1 = csub(v[1], v[3]);
-    double2 jb1 = inv ? make_double2(-b1.y, b1.x) : make_double2(b1.y, -b1.x);
-    v[0] = cadd(a0, b0);
-    v[2] = csub(a0, b0);
-    v[1] = cadd(a1, jb1);
-    v[3] = csub(a1, jb1);
-  } else {
-    double2 o[R];
-    const int m = n / R;
-#pragma unroll
-    for (int q = 0; q < R; ++q) {
-      double2 s = v[0];
-#pragma unroll
-      for (int r = 1; r < R; ++r) s = cadd(s, cmul(v[r], twid(tw, ((q * r) % R) * m, inv)));
-      o[q] = s;
-    }
-#pragma unroll
-    for (int q = 0; q < R; ++q) v[q] = o[q];
-  }
-}
-
-template <int R>
-__device__ inline void stockham_stage(const double2* __restrict__ src, double2* __restrict__ dst, int n,
-                                      int P, int Ns, const double2* __restrict__ tw, bool inv) {
-  const int m = n / R;
-  const int step = n / (Ns * R);
-  for (int idx = threadIdx.x; idx < P * m; idx += blockDim.x) {
-    const int k = idx / m;
-    const int j = idx - k * m;
-    const double2* s = src + k * n;
-    double2* d = dst + k * n;
-    const int kk = j % Ns;
-    double2 v[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      double2 x = s[j + r * m];
-      v[r] = r == 0 ? x : cmul(x, twid(tw, (r * kk * step) % n, inv));
-    }
-    small_dft<R>(v, tw, n, inv);
-    const int base = (j / Ns) * Ns * R + kk;
-#pragma unroll
-    for (int q = 0; q < R; ++q) d[base + q * Ns] = v[q];
-  }
-}
-
-// radix > 8: direct sum per output element
-__device__ inline void direct_stage(const double2* __restrict__ src, double2* __restrict__ dst, int n, int P,
-                                    int Ns, int R, const double2* __restrict__ tw, bool inv) {
-  const int m = n / R;
-  const int step = n / (Ns * R);
-  for (int idx = threadIdx.x; idx < P * n; idx += blockDim.x) {
-    const int k = idx / n;
-    const int rem = idx - k * n;
-    const int j = rem / R;
-    const int q = rem - j * R;
-    const double2* s = src + k * n;
-    const int kk = j % Ns;
-    double2 acc = make_double2(0.0, 0.0);
-    for (int r = 0; r < R; ++r) {
-      double2 x = s[j + r * m];
-      if (r) x = cmul(x, twid(tw, (int)(((long)r * kk * step) % n), inv));
-      acc = cadd(acc, cmul(x, twid(tw, ((q * r) % R) * m, inv)));
-    }
-    dst[k * n + (j / Ns) * Ns * R + kk + q * Ns] = acc;
-  }
-}
-
-// Transforms P pencils of length n held in a (ping-pong with b).  Returns
-// the buffer holding the result.  Ends with a barrier.
-__device__ double2* lds_fft(double2* a, double2* b, int n, int P, const FFTPlan& pl,
-                            const double2* __restrict__ tw, bool inv) {
-  int Ns = 1;
-  for (int s = 0; s < pl.nf; ++s) {
-    const int R = pl.fac[s];
-    switch (R) {
-      case 2: stockham_stage<2>(a, b, n, P, Ns, tw, inv); break;
-      case 3: stockham_stage<3>(a, b, n, P, Ns, tw, inv); break;
-      case 4: stockham_stage<4>(a, b, n, P, Ns, tw, inv); break;
-      case 5: stockham_stage<5>(a, b, n, P, Ns, tw, inv); break;
-      case 7: stockham_stage<7>(a, b, n, P, Ns, tw, inv); break;
-      default: direct_stage(a, b, n, P, Ns, R, tw, inv); break;
-    }
-    __syncthreads();
-    double2* t = a;
-    a = b;
-    b = t;
-    Ns *= R;
-  }
-  return a;
-}
-
-// ---------------------------------------------------------------------------
-// Self-energy pass.  One workgroup: row q (t' = tmin + q) x P pencils along
-// `axis`.  See SigmaArgs for the flags.
-// ---------------------------------------------------------------------------
-__device__ inline int site_of(const SigmaArgs& a, int pencil, int j) {
-  // dims (nx, ny, nz); pencil enumerates the two non-transform coordinates
-  if (a.axis == 0) {
-    const int iy = pencil % a.ny, iz = pencil / a.ny;
-    return j + a.nx * (iy + a.ny * iz);
-  } else if (a.axis == 1) {
-    const int ix = pencil % a.nx, iz = pencil / a.nx;
-    return ix + a.nx * (j + a.ny * iz);
-  } else {
-    const int ix = pencil % a.nx, iy = pencil / a.nx;
-    return ix + a.nx * (iy + a.ny * j);
-  }
-}
-
-__device__ inline int neg_site(const SigmaArgs& a, int s) {
-  const int ix = s % a.nx;
-  const int iy = (s / a.nx) % a.ny;
-  const int iz = s / (a.nx * a.ny);
-  const int jx = (a.nx - ix) % a.nx, jy = (a.ny - iy) % a.ny, jz = (a.nz - iz) % a.nz;
-  return jx + a.nx * (jy + a.ny * jz);
-}
-
-__global__ __launch_bounds__(256) void sigma_pass(SigmaArgs a) {
-  extern __shared__ double2 lds[];
-  const int n = a.n;
-  const int P = a.P;
-  double2* A = lds;
-  double2* B = lds + P * n;
-  const int q = blockIdx.y;
-  if (q >= a.st->L) return;  // rows t' = tmin + q, q < L, are live
-  const int pen0 = blockIdx.x * P;
-  const int tp = a.st->tmin + q;
-  const int s_tm1 = a.st->s_tm1;
-  const int slot = (tp - 1) % a.N;
-  const size_t rowoff = (size_t)q * a.V;
-  const bool contiguous = a.axis == 0;
-
-  // ---- load ----
-  for (int e = threadIdx.x; e < P * n; e += blockDim.x) {
-    int k, j;
-    if (contiguous) {
-      k = e / n;
-      j = e - k * n;
-    } else {
-      j = e / P;
-      k = e - j * P;
-    }
-    const int pencil = pen0 + k;
-    double2 z = make_double2(0.0, 0.0);
-    if (pencil < a.npencils) {
-      const int s = site_of(a, pencil, j);
-      if (a.flags & SIGMA_GATHER) {
-        // physical F(t-1,t') and rho(t-1,t'); rho sign from the slot order
-        const long pr = pair_off(s_tm1, slot, a.N);
-        const double sg = s_tm1 >= slot ? 1.0 : -1.0;
-        const int s2 = neg_site(a, s);
-        const double* h1 = a.H + hoff(s / MB, pr, s % MB, a.NP);
-        const double* h2 = a.H + hoff(s2 / MB, pr, s2 % MB, a.NP);
-        // real(rfft(X)) only sees the inversion-even part of X
-        z.x = 0.5 * (h1[0] + h2[0]);
-        z.y = 0.5 * (h1[1] + h2[1]) * sg;
-      } else {
-        z = a.W[rowoff + s];
-      }
-    }
-    A[k * n + j] = z;
-  }
-  __syncthreads();
-
-  // ---- transform(s) ----
-  double2* res = lds_fft(A, B, n, P, a.plan, a.tw, (a.flags & SIGMA_INVERSE) != 0);
-  if (a.flags & SIGMA_SUNSET) {
-    double2* other = res == A ? B : A;
-    // quantum sunset; the classical one drops the rho^2 terms
-    const double qF = a.classical ? 0.0 : 0.75, qr = a.classical ? 0.0 : 1.0 / 12.0;
-    for (int e = threadIdx.x; e < P * n; e += blockDim.x) {
-      const double2 z = res[e];
-      const double Fx = z.x, rx = z.y;
-      const double FF = Fx * Fx, rr = rx * rx;
-      res[e] = make_double2(Fx * (FF - qF * rr), rx * (FF - qr * rr));
-    }
-    __syncthreads();
-    res = lds_fft(res, other, n, P, a.plan, a.tw, true);
-  }
-
-  // ---- store ----
-  for (int e = threadIdx.x; e < P * n; e += blockDim.x) {
-    int k, j;
-    if (contiguous) {
-      k = e / n;
-      j = e - k * n;
-    } else {
-      j = e / P;
-      k = e - j * P;
-    }
-    const int pencil = pen0 + k;
-    if (pencil >= a.npencils) continue;
-    const int s = site_of(a, pencil, j);
-    const double2 z = res[k * n + j];
-    if (a.flags & SIGMA_SCATTER) {
-      double* o = a.S + soff(s / MB, slot, s % MB, a.N);
-      o[0] = a.preF * z.x;
-      o[1] = a.preR * z.y;
-    } else {
-      a.W[rowoff + s] = z;
-    }
-  }
-}
 
 // ---------------------------------------------------------------------------
 // Hartree mass: m2 = Mass2 + H ivol sum_p F(t-1,t-1;p)

@@ -126,12 +126,8 @@ int device_setup(int dev) {
   if (se != hipSuccess || !ptr)
     return fail(KB_ERR_HIP, "sunset: no device address for the scratch array: %s", hipGetErrorString(se));
   g_scratch[dev] = static_cast<char*>(ptr);
-  // every compiled length and the runtime-length instantiation
-  static const int lengths[] = {8, 16, 24, 32, 40, 48, 64, 1};
-  for (int n : lengths) {
-    hipError_t e = sigma_planes_prepare(n);
-    if (e != hipSuccess) return fail(KB_ERR_HIP, "sunset: plane kernel set-up failed: %s", hipGetErrorString(e));
-  }
+  hipError_t e = sigma_prepare();
+  if (e != hipSuccess) return fail(KB_ERR_HIP, "sunset: transform pass set-up failed: %s", hipGetErrorString(e));
   g_ready[dev] = true;
   return KB_OK;
 }
@@ -164,7 +160,7 @@ int run_sunset(const kb_params* p, int nrows, const double* F, const double* rho
   a.Sigrout = Sigr;
   a.rows = nrows;
   a.classical = p->pexp == KB_PEXP_LAMBDA_NLO_CLASSICAL;
-  e = launch_sigma_planes_plain(a, st);
+  e = launch_sigma_stage(a, SG_PLAIN, nrows, st);
   if (e != hipSuccess) return fail(KB_ERR_HIP, "sunset: plane kernel launch failed: %s", hipGetErrorString(e));
   return KB_OK;
 }
