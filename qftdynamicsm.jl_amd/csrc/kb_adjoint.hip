@@ -183,7 +183,6 @@ __global__ void adj_slide_kernel(double* __restrict__ H, double* __restrict__ Hb
   if (tape) st2(H + o, ld2(tape + ((((size_t)mb * N) + x) * MB + lane) * 2));
 }
 
-__global__ void adj_state_kernel(StepState* st, int t, int N) { *st = state_of_step(t, N); }
 
 // dL/dF of F(T-1,T-1), F(T,T-1), F(T,T) for L = sum wgt n(T); n as
 // createMeasurement (Measurement.jl:38-59) with its stability clamp
@@ -1014,15 +1013,18 @@ int reverse_step(kb_ctx* c, int t, int T, int npend, bool apply) {
   int rc;
   {
     StageTimer tm(c, 4);
-    hipLaunchKernelGGL(adj_state_kernel, dim3(1), dim3(1), 0, c->stream, c->st_dev, t, N);
+    // the state of the step being reversed, M^2(t) and sum_p F(t-1,t-1;p)
+    const double H = c->p.Lambda * (double)(c->p.ONgroup + 2) / (6.0 * (double)c->p.ONgroup);
+    HartreeArgs h = hartree_args(c);
+    h.t = t;
+    h.hfac = H / (double)c->Vl;
+    h.wgt = nullptr;
+    h.out = s->m2r + (t & 1) * 2;
+    h.sum_out = h.out + 1;
+    hipLaunchKernelGGL(hartree_step_kernel, dim3(hartree_groups(c->V)), dim3(HARTREE_THREADS), 0, c->stream, h, nullptr,
+                       1);
     LAUNCHCHK(c);
     if (nlo && (rc = launch_sigma(c, s->X, s->Sring[t % AK]))) return rc;
-    const double H = c->p.Lambda * (double)(c->p.ONgroup + 2) / (6.0 * (double)c->p.ONgroup);
-    // M^2(t) and sum_p F(t-1,t-1;p) of the step being reversed (st_dev holds its state)
-    double* m2t = s->m2r + (t & 1) * 2;
-    hipLaunchKernelGGL(hartree_step_kernel, dim3(hartree_groups(c->V)), dim3(HARTREE_THREADS), 0, c->stream, c->H,
-                       c->NP, c->V, N, c->st_dev, H / (double)c->Vl, c->p.Mass2, nullptr, m2t, c->hpart, m2t + 1);
-    LAUNCHCHK(c);
     set_pending(c, a, t + 1, nlo ? npend : 0);
     launch_row<0>(a.npend, dim3(c->NB), c->stream, a);
     LAUNCHCHK(c);

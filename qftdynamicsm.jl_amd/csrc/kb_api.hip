@@ -376,11 +376,25 @@ hipError_t launch_memint(int tile, unsigned grid, int maxN, hipStream_t s, const
 
 size_t memint_lds(int N) { return sizeof(double) * 2 * (size_t)N * MB; }
 
+HartreeArgs hartree_args(const kb_ctx* c) {
+  HartreeArgs a{};
+  a.H = c->H;
+  a.wgt = c->wgt_dev;
+  a.out = c->m2;
+  a.part = c->hpart;
+  a.st = c->st_dev;
+  a.NP = c->NP;
+  a.V = c->V;
+  a.N = c->N;
+  a.hfac = hartree_prefactor(c) * (1.0 / (double)c->Vl);
+  a.Mass2 = c->p.Mass2;
+  return a;
+}
+
+// advances st_dev
 int launch_hartree_step(kb_ctx* c) {
-  const double H = hartree_prefactor(c);
-  const double hfac = H * (1.0 / (double)c->Vl);
-  hipLaunchKernelGGL(hartree_step_kernel, dim3(hartree_groups(c->V)), dim3(HARTREE_THREADS), 0, c->stream, c->H, c->NP,
-                     c->V, c->N, c->st_dev, hfac, c->p.Mass2, c->wgt_dev, c->m2, c->hpart, nullptr);
+  hipLaunchKernelGGL(hartree_step_kernel, dim3(hartree_groups(c->V)), dim3(HARTREE_THREADS), 0, c->stream,
+                     hartree_args(c), nullptr, 1);
   LAUNCHCHK(c);
   return KB_OK;
 }
@@ -419,18 +433,16 @@ int launch_memint_step(kb_ctx* c) {
 // argument is step-invariant, the window comes from st_dev.
 int enqueue_step(kb_ctx* c) {
   int rc;
-  hipLaunchKernelGGL(advance_kernel, dim3(1), dim3(64), 0, c->stream, c->stptr_dev, c->N_dev, 1);
-  LAUNCHCHK(c);
+  {
+    StageTimer st(c, 2);
+    if ((rc = launch_hartree_step(c))) return rc;
+  }
   if (sunset_expansion(c->p.pexp)) {
     StageTimer st(c, 1);
     if ((rc = launch_sigma(c))) return rc;
   } else if (c->p.pexp == KB_PEXP_NINVERSE_NLO) {
     StageTimer st(c, 1);
     if ((rc = launch_ninv_stage(c))) return rc;
-  }
-  {
-    StageTimer st(c, 2);
-    if ((rc = launch_hartree_step(c))) return rc;
   }
   {
     StageTimer st(c, 0);
@@ -853,10 +865,7 @@ static int create_ctx(const kb_params* p, bool sym, kb_ctx** out) {
     with((void**)&c->flag, nullptr, 4 * sizeof(int));
     with((void**)&c->wg0_dev, nullptr, sizeof(int));
     with((void**)&c->st_dev, &c->st, sizeof(StepState));
-    with((void**)&c->N_dev, &c->N, sizeof(int));
-    // these two hold device addresses: filled in once the arena has one
-    const size_t stptr_off = used;
-    with((void**)&c->stptr_dev, nullptr, sizeof(StepState*));
+    // holds device addresses: filled in once the arena has one
     const size_t margs_off = used;
     with((void**)&c->margs_dev, nullptr, sizeof(MemintArgs));
     if (sym || c->hstage_n == 2 * HSTAGE_MAX) place((void**)&c->modes, (size_t)6 * c->V * sizeof(double));
@@ -866,7 +875,6 @@ static int create_ctx(const kb_params* p, bool sym, kb_ctx** out) {
     if ((rc = dmalloc(c, &c->arena, used))) return fail(rc);
     for (const Part& q : parts) *q.ptr = static_cast<char*>(c->arena) + q.off;
     c->items = c->items_r[1];
-    std::memcpy(image.data() + stptr_off, &c->st_dev, sizeof(StepState*));
     const MemintArgs ma = memint_args(c);
     std::memcpy(image.data() + margs_off, &ma, sizeof(MemintArgs));
     if (hipMemcpy(c->arena, image.data(), image.size(), hipMemcpyHostToDevice) != hipSuccess) return fail(KB_ERR_HIP);
@@ -1617,12 +1625,12 @@ struct kb_ens {
   std::vector<hipEvent_t> join;
   std::vector<int> lane;
   hipEvent_t fork = nullptr;
-  StepState** stptr_dev = nullptr;
-  int* N_dev = nullptr;
   // memory-integral argument tables, runs ordered by lane: lane j owns runs
   // [lrun[j], lrun[j+1]) and lwg[j] workgroups; wg_dev holds each run's
   // first workgroup over all lanes (one pooled launch), lwg_dev within its
   // lane (one launch per lane)
+  HartreeArgs* hargs_dev = nullptr;
+  int hartree_wg = 0;
   MemintArgs* margs_dev = nullptr;
   int* wg_dev = nullptr;
   int* lwg_dev = nullptr;
@@ -1672,7 +1680,7 @@ void ens_free(kb_ens* e) {
       kb_destroy(c);
     }
   }
-  for (void* p : {(void*)e->stptr_dev, (void*)e->N_dev, (void*)e->margs_dev, (void*)e->wg_dev, (void*)e->lwg_dev})
+  for (void* p : {(void*)e->hargs_dev, (void*)e->margs_dev, (void*)e->wg_dev, (void*)e->lwg_dev})
     if (p) (void)hipFree(p);
   for (auto& ev : e->pending) {
     (void)hipEventDestroy(ev.a);
@@ -1719,23 +1727,23 @@ int ens_make_lanes(kb_ens* e) {
   return KB_OK;
 }
 
-// one ensemble step: advance all windows; each member's self-energy and
-// Hartree kernels on its lane; the memory integrals of all members in one
+// one ensemble step: the Hartree masses (and advanced windows) of all members
+// in one launch; each member's self-energy on its lane; the memory integrals of all members in one
 // launch after the lanes have joined, or (lane_integrals) one per lane
 // after that lane's stages
 int ens_enqueue(kb_ens* e) {
-  const int nr = (int)e->m.size();
-  hipLaunchKernelGGL(advance_kernel, dim3(1), dim3(64 * ((nr + 63) / 64)), 0, e->stream, e->stptr_dev, e->N_dev, nr);
+  hipLaunchKernelGGL(hartree_step_kernel, dim3(e->hartree_wg), dim3(HARTREE_THREADS), 0, e->stream,
+                     hartree_args(e->m[0]), e->hargs_dev, (int)e->m.size());
   hipError_t err = hipGetLastError();
-  if (err != hipSuccess) return ens_err(e, KB_ERR_HIP, "advance launch failed: %s", hipGetErrorString(err));
+  if (err != hipSuccess) return ens_err(e, KB_ERR_HIP, "Hartree launch failed: %s", hipGetErrorString(err));
   const bool forked = !e->side.empty();
   if (forked) {
     err = hipEventRecord(e->fork, e->stream);
     for (size_t j = 1; j < e->side.size() && err == hipSuccess; ++j) err = hipStreamWaitEvent(e->side[j], e->fork, 0);
     if (err != hipSuccess) return ens_err(e, KB_ERR_HIP, "fork: %s", hipGetErrorString(err));
   }
-  // per lane: its members' self-energy and Hartree kernels, then (with
-  // lane_integrals) the memory integral over its members
+  // per lane: its members' self-energies, then (with lane_integrals) the
+  // memory integral over its members
   int rc = KB_OK;
   const int nl = (int)e->lwg.size();
   for (int j = 0; j < nl && rc == KB_OK; ++j) {
@@ -1748,8 +1756,6 @@ int ens_enqueue(kb_ens* e) {
         rc = ens_err(e, rc, "member self-energy: %s", c->err.c_str());
       else if (c->p.pexp == KB_PEXP_NINVERSE_NLO && (rc = launch_ninv_stage(c)))
         rc = ens_err(e, rc, "member 1/N self-energy: %s", c->err.c_str());
-      else if ((rc = launch_hartree_step(c)))
-        rc = ens_err(e, rc, "member Hartree: %s", c->err.c_str());
     }
     if (rc == KB_OK && e->lane_integrals && e->lwg[j] > 0) {
       // one shape for all members (their item tables follow its row height)
@@ -1769,7 +1775,7 @@ int ens_enqueue(kb_ens* e) {
   }
   if (rc) return rc;
   if (!e->lane_integrals) {
-    err = launch_memint(e->tile, e->total_wg, e->maxN, e->stream, e->margs_dev, e->wg_dev, nr);
+    err = launch_memint(e->tile, e->total_wg, e->maxN, e->stream, e->margs_dev, e->wg_dev, (int)e->m.size());
     if (err != hipSuccess) return ens_err(e, KB_ERR_HIP, "memint launch failed: %s", hipGetErrorString(err));
   }
   return KB_OK;
@@ -1923,20 +1929,18 @@ int kb_ens_create_sym(const kb_params* params, const int* symmetric, int nruns, 
   if (hipSetDevice(e->device) != hipSuccess) return fail(KB_ERR_HIP);
   if (hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking) != hipSuccess) return fail(KB_ERR_HIP);
   if (ens_make_lanes(e) != KB_OK) return fail(KB_ERR_HIP);
-  std::vector<StepState*> sp;
-  std::vector<int> Ns;
   for (auto* c : e->m) {
     (void)hipStreamSynchronize(c->stream);
     c->stream = e->stream;
     c->in_ensemble = true;
-    sp.push_back(c->st_dev);
-    Ns.push_back(c->N);
   }
-  if (hipMalloc((void**)&e->stptr_dev, sizeof(StepState*) * nruns) != hipSuccess ||
-      hipMalloc((void**)&e->N_dev, sizeof(int) * nruns) != hipSuccess)
-    return fail(KB_ERR_OOM);
-  if (hipMemcpy(e->stptr_dev, sp.data(), sizeof(StepState*) * nruns, hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(e->N_dev, Ns.data(), sizeof(int) * nruns, hipMemcpyHostToDevice) != hipSuccess)
+  std::vector<HartreeArgs> ha;
+  for (auto* c : e->m) {
+    ha.push_back(hartree_args(c));
+    e->hartree_wg += hartree_groups(c->V);
+  }
+  if (hipMalloc((void**)&e->hargs_dev, sizeof(HartreeArgs) * nruns) != hipSuccess) return fail(KB_ERR_OOM);
+  if (hipMemcpy(e->hargs_dev, ha.data(), sizeof(HartreeArgs) * nruns, hipMemcpyHostToDevice) != hipSuccess)
     return fail(KB_ERR_HIP);
   if (int rc = ens_upload_tables(e)) return fail(rc);
   e->lane_integrals = e->side.size() > 1;

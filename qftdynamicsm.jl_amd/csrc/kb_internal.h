@@ -92,8 +92,6 @@ struct kb_ctx {
   int Mp = 0, Kp = 0, ldg = 0;
   // device-resident step state and launch tables (graph-capturable steps)
   qftkb::StepState* st_dev = nullptr;
-  qftkb::StepState** stptr_dev = nullptr;  // {st_dev}
-  int* N_dev = nullptr;
   qftkb::MemintArgs* margs_dev = nullptr;
   int* wg0_dev = nullptr;  // {0}
   bool use_graph = false;
@@ -180,6 +178,7 @@ inline bool has_sigma(const kb_ctx* c) {
 // orbits of the lattice's cubic group (axis permutations, reflections
 // n -> Nx - n): lattice site -> orbit, and orbit -> its first site
 void cubic_orbits(int Nx, int sdim, std::vector<int>& orbit_of, std::vector<int>& rep_site);
+qftkb::HartreeArgs hartree_args(const kb_ctx* c);
 // the kernels of one forward step (the window in c->st_dev is advanced first)
 int enqueue_step(kb_ctx* c);
 size_t memint_lds(int N);

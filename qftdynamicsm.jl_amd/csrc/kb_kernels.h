@@ -18,7 +18,7 @@ struct FFTPlan {
 };
 
 // Window of the step being taken, after expandSimData! (SimDataStruct.jl:
-// 262-278).  Kept in device memory and advanced by advance_kernel, so a
+// 262-278).  Kept in device memory and advanced by hartree_step_kernel, so a
 // step's kernels have step-invariant arguments and can be replayed from a
 // captured hipGraph.
 struct StepState {
@@ -182,17 +182,31 @@ struct MeasArgs {
 // wgt: sites each stored site stands for (orbit storage), NULL = 1
 __global__ void hartree_kernel(const double* H, long NP, int V, long pair, double hfac, double Mass2,
                                const double* wgt, double* out);
-// Hartree mass of the step being taken: F(t-1,t-1) from *st; one workgroup
-// of HARTREE_THREADS per HARTREE_SITES sites, part: hartree_groups(V)
-// partial sums followed by a zeroed counter (hartree_part_doubles(V) doubles);
-// sum_out (may be null) receives the weighted sum of F(t-1,t-1) itself
-constexpr int HARTREE_THREADS = 256;
-constexpr int HARTREE_LOADS = 8;
+// First kernel of a step: *st becomes the state of step t, or (t = 0) the
+// next one, and out the Hartree mass from its F(t-1,t-1).  hartree_groups(V)
+// workgroups of HARTREE_THREADS; part: their partial sums followed by a zeroed
+// counter (hartree_part_doubles(V) doubles); sum_out (may be null) receives
+// the weighted sum of F(t-1,t-1) itself.  Several runs come as a table, each
+// with its own workgroups, one after another.
+struct HartreeArgs {
+  const double* H;
+  const double* wgt;
+  double *out, *part, *sum_out;
+  StepState* st;
+  long NP;
+  int V, N, t;
+  double hfac, Mass2;
+};
+constexpr int HARTREE_THREADS = 1024;
+constexpr int HARTREE_LOADS = 4;
 constexpr int HARTREE_SITES = HARTREE_THREADS * HARTREE_LOADS;
-inline int hartree_groups(int V) { return (V + HARTREE_SITES - 1) / HARTREE_SITES; }
+constexpr int HARTREE_GROUPS = 96;  // at most
+__host__ __device__ inline int hartree_groups(int V) {
+  const int g = (V + HARTREE_SITES - 1) / HARTREE_SITES;
+  return g < HARTREE_GROUPS ? g : HARTREE_GROUPS;
+}
 inline size_t hartree_part_doubles(int V) { return (size_t)hartree_groups(V) + 2; }
-__global__ void hartree_step_kernel(const double* H, long NP, int V, int N, const StepState* st, double hfac,
-                                    double Mass2, const double* wgt, double* out, double* part, double* sum_out);
+__global__ void hartree_step_kernel(HartreeArgs one, const HartreeArgs* runs, int nruns);
 // one launch over all runs: workgroups [wg_start[r], wg_start[r+1]) belong to run r
 template <int ROWS, int B, int TPB>
 __global__ void memint_step(const MemintArgs* runs, const int* wg_start, int nruns);
@@ -225,7 +239,6 @@ struct MemintVariant {
 constexpr int NMEMINT_VARIANTS = 13;
 extern const MemintVariant kMemintVariants[NMEMINT_VARIANTS];
 constexpr int MEMINT_ROW_CHOICES[3] = {32, 64, 128};  // item tables kept per context
-__global__ void advance_kernel(StepState* const* states, const int* Ns, int nruns);
 __global__ void measure_kernel(MeasArgs a);
 __global__ void measure_finish(MeasArgs a, int groups);
 __global__ void expand_kernel(const double* src, int V, const int* smap, int Vl, int narr, double* dst);

@@ -39,66 +39,71 @@ __global__ __launch_bounds__(1024) void hartree_kernel(const double* __restrict_
   }
 }
 
-// One workgroup per HARTREE_SITES sites, HARTREE_LOADS loads in flight per
-// thread (the diagonal entries lie one per 128-byte line of every site
-// block, so a single workgroup is latency-bound).  Each workgroup writes its
-// partial sum; the last one to finish (an agent-scope counter: the
-// workgroups sit on different XCDs) adds the partials in workgroup order, so
-// the result does not depend on which one that is, and resets the counter.
-__global__ __launch_bounds__(HARTREE_THREADS) void hartree_step_kernel(const double* __restrict__ H, long NP, int V,
-                                                                       int N, const StepState* __restrict__ st,
-                                                                       double hfac, double Mass2,
-                                                                       const double* __restrict__ wgt,
-                                                                       double* __restrict__ out, double* part,
-                                                                       double* __restrict__ sum_out) {
+// A step's first kernel: its Hartree mass, and its window state, which every
+// workgroup works out from the stored one and the last workgroup stores.  (A
+// launch of its own for the state took 4 us of a step.)
+//
+// Bound by latency, HARTREE_LOADS loads in flight per thread; past some 2^18
+// sites by the counter, some 35 ns per workgroup, hence at most HARTREE_GROUPS
+// of them (112^3: 686 took 25 us).  Each workgroup writes its
+// partial sum; the last one to finish (an agent-scope counter: the workgroups
+// sit on different XCDs) adds the partials in workgroup order, so the result
+// does not depend on which one that is, and resets the counter.
+// An ensemble's runs share one launch, like memint_step_runs.
+__global__ __launch_bounds__(HARTREE_THREADS) void hartree_step_kernel(HartreeArgs one,
+                                                                       const HartreeArgs* __restrict__ runs,
+                                                                       int nruns) {
   __shared__ double red[HARTREE_THREADS / 64];
   __shared__ int is_last;
-  const long pair = pair_off(st->s_tm1, st->s_tm1, N);  // F(t-1,t-1), Evolution.jl:945
-  const int G = gridDim.x;
-  double v[HARTREE_LOADS];
-#pragma unroll
-  for (int u = 0; u < HARTREE_LOADS; ++u) {
-    const int p = blockIdx.x * HARTREE_SITES + u * HARTREE_THREADS + threadIdx.x;
-    v[u] = p < V ? (wgt ? wgt[p] : 1.0) * H[hoff(p / MB, pair, p % MB, NP)] : 0.0;
+  HartreeArgs a = one;
+  int group = blockIdx.x;
+  if (nruns > 1) {
+    int run = 0;
+    while (group >= hartree_groups(runs[run].V)) group -= hartree_groups(runs[run++].V);
+    a = runs[run];
   }
+  const int N = a.N, V = a.V, G = hartree_groups(V);
+  StepState s = a.t ? state_of_step(a.t, N) : *a.st;
+  if (!a.t) advance_state(s, N);
+  const long pair = pair_off(s.s_tm1, s.s_tm1, N);  // F(t-1,t-1), Evolution.jl:945
+  double* part = a.part;
   double acc = 0.0;
+  for (int base = group * HARTREE_SITES; base < V; base += G * HARTREE_SITES) {
+    double v[HARTREE_LOADS];
 #pragma unroll
-  for (int u = 0; u < HARTREE_LOADS; ++u) acc += v[u];
+    for (int u = 0; u < HARTREE_LOADS; ++u) {
+      const int p = base + u * HARTREE_THREADS + threadIdx.x;
+      v[u] = p < V ? (a.wgt ? a.wgt[p] : 1.0) * a.H[hoff(p / MB, pair, p % MB, a.NP)] : 0.0;
+    }
+#pragma unroll
+    for (int u = 0; u < HARTREE_LOADS; ++u) acc += v[u];
+  }
   for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
   __syncthreads();
-  unsigned* count = reinterpret_cast<unsigned*>(part + G);
-  if (threadIdx.x == 0) {
-    double b = 0.0;
-    for (int w = 0; w < HARTREE_THREADS / 64; ++w) b += red[w];
-    part[blockIdx.x] = b;
-    is_last = __hip_atomic_fetch_add(count, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)G - 1;
+  if (G > 1) {
+    unsigned* count = reinterpret_cast<unsigned*>(part + G);
+    if (threadIdx.x == 0) {
+      double b = 0.0;
+      for (int w = 0; w < HARTREE_THREADS / 64; ++w) b += red[w];
+      part[group] = b;
+      is_last = __hip_atomic_fetch_add(count, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)G - 1;
+      if (is_last) __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (!is_last) return;
+    // the partials in a fixed order
+    double h = (int)threadIdx.x < G ? part[threadIdx.x] : 0.0;
+    for (int o = 32; o > 0; o >>= 1) h += __shfl_xor(h, o);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = h;
+    __syncthreads();
   }
-  __syncthreads();
-  if (!is_last) return;
-  // the partials in a fixed order: thread k takes k, k + T, ..., then the
-  // same tree as above
-  double h = 0.0;
-  for (int g = threadIdx.x; g < G; g += HARTREE_THREADS) h += part[g];
-  for (int o = 32; o > 0; o >>= 1) h += __shfl_xor(h, o);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = h;
-  __syncthreads();
   if (threadIdx.x == 0) {
     double tot = 0.0;
     for (int w = 0; w < HARTREE_THREADS / 64; ++w) tot += red[w];
-    out[0] = tot * hfac + Mass2;
-    if (sum_out) sum_out[0] = tot;
-    __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
-}
-
-__global__ void advance_kernel(StepState* const* states, const int* Ns, int nruns) {
-  const int r = threadIdx.x;
-  if (r < nruns) {
-    StepState s = *states[r];
-    advance_state(s, Ns[r]);
-    *states[r] = s;
+    a.out[0] = tot * a.hfac + a.Mass2;
+    if (a.sum_out) a.sum_out[0] = tot;
+    *a.st = s;
   }
 }
 
