@@ -315,7 +315,7 @@ int kb_adj_get_entry(kb_ctx *ctx, int which, int i, int j, double *out);
  * calcSelfEnergyattp! (TwoPIScalar_Evolution.jl:25-31, LambdaNLOquantum) on
  * lattices that the caller holds in device memory, without a context: for
  * each of nrows rows q, Sigr(q) and SigF(q) of the pair F(q), rho(q) (rho
- * physical), by the plane kernels of the KB step with the same twiddles, so
+ * physical), by the transforms of the KB step with the same twiddles, so
  * a row gives the same bits as kb_step's self-energy stage.  Rows are V =
  * Nx^sdim doubles at q*V, column-major sites; F, rho, SigF and Sigr are
  * device pointers on p->device.  Only Nx, sdim, ONgroup, Lambda, pexp
@@ -324,7 +324,7 @@ int kb_adj_get_entry(kb_ctx *ctx, int which, int i, int j, double *out);
  * outputs may not overlap the inputs or each other.
  *
  * The workspace is caller-owned device memory of kb_sunset_workspace_bytes
- * (4 KiB of twiddles, plus nrows * Nx^2 (Nx/2 + 1) complex values in 3D: the
+ * (4 KiB, plus nrows * Nx^2 (Nx/2 + 1) complex values in 3D: the
  * half space of each row's transforms), 256-byte
  * aligned.  Kernels are enqueued on `stream` (a hipStream_t; NULL = the
  * device's null stream) and the call returns without waiting.  Errors are
@@ -341,7 +341,7 @@ int kb_sunset(const kb_params *p, int nrows, const double *F, const double *rho,
  * a 64 MiB device array inside the library, one per device, held until the
  * process ends: KB_ERR_ARG when kb_sunset_workspace_bytes of the request
  * exceeds 64 MiB (more than 31 rows of 64^3, 72 of 48^3, 240 of 32^3; 1D and
- * 2D lattices need only the 4 KiB of twiddles).
+ * 2D lattices need only the 4 KiB).
  * Every call on one device shares that array, so calls that overlap in time
  * on one device (other streams, other threads) race; the results equal
  * kb_sunset's. */

@@ -17,6 +17,7 @@
 
 #include "../../include/qftkb.h"
 #include "kb_internal.h"
+#include "kb_twiddles.h"
 
 #ifndef KB_MSPLIT_MAX
 #define KB_MSPLIT_MAX 8
@@ -54,8 +55,14 @@ int seterr(kb_ctx* c, int code, const char* fmt, ...) {
 inline int slot_of(const kb_ctx* c, int t) { return (t - 1) % c->N; }
 inline bool inwin(const kb_ctx* c, int t) { return c->st.tmin <= t && t <= c->st.tmax; }
 
+// (kb_sunset's table for its lengths: its rows have a step's bits)
 void fft_twiddles(int n, double2* out) {
-  for (int k = 0; k < n; ++k) {
+  static constexpr TwiddleTable table = make_twiddles();
+  for (int k = 0; k < n && n <= TWIDDLE_MAX; ++k) {
+    const double* w = table.v + 2 * (twiddle_start(n) + k);
+    out[k] = make_double2(w[0], w[1]);
+  }
+  for (int k = n <= TWIDDLE_MAX ? n : 0; k < n; ++k) {
     long double a = -2.0L * 3.14159265358979323846264338327950288L * (long double)k / (long double)n;
     out[k] = make_double2((double)cosl(a), (double)sinl(a));
   }

@@ -1,14 +1,13 @@
 // kb_lattice.hip -- context-free entry points on lattices that the caller
 // keeps in device memory: the sunset self-energies of calcSelfEnergyattp!
 // (TwoPIScalar_Evolution.jl:25-31) for rows of F and rho, computed by the
-// plane kernels of the KB step (kb_sigma.hip, mode SG_PLAIN) with the same
+// passes of the KB step (kb_sigma_impl.h, mode SG_PLAIN) with the same
 // twiddles as a context, so a row gives the same bits as the step's
 // self-energy stage.
 //
 // Device memory: the caller's input and output rows, plus a workspace that
-// holds the twiddle table (the first WS_TWIDDLE_BYTES) and, for 3D lattices,
-// half a complex lattice per row (the planes z in [0, Nx/2]) for the
-// transforms between the plane passes.
+// holds, for 3D lattices, half a complex lattice per row (the planes z in
+// [0, Nx/2]) for the transforms between the passes, behind WS_HEAD_BYTES.
 // kb_sunset takes the workspace from the caller; kb_sunset_noalloc uses the
 // file-scope device array `scratch` below (SCRATCH_BYTES on every device the
 // library runs on, held until the process ends), so it allocates nothing.
@@ -22,6 +21,7 @@
 
 #include "../../include/qftkb.h"
 #include "kb_internal.h"
+#include "kb_twiddles.h"
 
 using namespace qftkb;
 using namespace qftkb_host;
@@ -41,34 +41,30 @@ int fail(int code, const char* fmt, ...) {
   return code;
 }
 
-constexpr int NX_MAX = 64;                 // the plane kernels' largest lattice
-constexpr size_t WS_TWIDDLE_BYTES = 4096;  // >= NX_MAX complex values, keeps the rows 256-byte aligned
+constexpr int NX_MAX = TWIDDLE_MAX;        // the largest lattice
+constexpr size_t WS_HEAD_BYTES = 4096;     // not used (callers' workspaces hold it all the same)
 constexpr int MAX_DEVICES = 64;
 constexpr int MAX_ROWS = 65535;            // grid rows of one launch
 
 // kb_sunset_noalloc's workspace.  In host code `scratch` names a host-side
 // stand-in, not a device address: only the address that hipGetSymbolAddress
 // returns for the current device (kept per device in g_scratch) is used.
-// Nothing in it needs clearing: every call writes the twiddles and the rows
+// Nothing in it needs clearing: every call writes the rows
 // before reading them.  Calls on one device share it and must not overlap.
 constexpr size_t SCRATCH_BYTES = size_t(64) << 20;
 static __device__ __align__(256) char scratch[SCRATCH_BYTES];
 
-// the host twiddle table, passed by value to the kernel that stores it
-struct Twiddles {
-  double2 w[NX_MAX];
-};
+// The twiddles of every length, in the code object: filling a table in the
+// workspace took a launch of 3 us, a quarter of a call on 8^3.
+// (not const: a constant that no device code names is left out of the device
+// image, and its address could not be asked for)
+static __device__ TwiddleTable twiddle_table = make_twiddles();
 
-__global__ void put_twiddles(Twiddles t, double2* dst, int n) {
-  const int k = threadIdx.x;
-  if (k < n) dst[k] = t.w[k];
-}
-
-// rows of complex values between the plane passes (3D only): the half space
+// rows of complex values between the passes (3D only): the half space
 // z in [0, Nx/2] of each row
 size_t workspace_bytes(const kb_params* p, int nrows) {
   const size_t half = (size_t)p->Nx * p->Nx * (p->Nx / 2 + 1);
-  return WS_TWIDDLE_BYTES + (p->sdim == 3 ? (size_t)nrows * half * sizeof(double2) : 0);
+  return WS_HEAD_BYTES + (p->sdim == 3 ? (size_t)nrows * half * sizeof(double2) : 0);
 }
 
 int check_params(const kb_params* p, int nrows) {
@@ -117,6 +113,7 @@ struct DeviceScope {
 std::mutex g_setup_mu;
 bool g_ready[MAX_DEVICES] = {};
 char* g_scratch[MAX_DEVICES] = {};
+const double2* g_twiddles[MAX_DEVICES] = {};
 
 int device_setup(int dev) {
   std::lock_guard<std::mutex> lk(g_setup_mu);
@@ -126,25 +123,23 @@ int device_setup(int dev) {
   if (se != hipSuccess || !ptr)
     return fail(KB_ERR_HIP, "sunset: no device address for the scratch array: %s", hipGetErrorString(se));
   g_scratch[dev] = static_cast<char*>(ptr);
+  se = hipGetSymbolAddress(&ptr, HIP_SYMBOL(twiddle_table));
+  if (se != hipSuccess || !ptr)
+    return fail(KB_ERR_HIP, "sunset: no device address for the twiddles: %s", hipGetErrorString(se));
+  g_twiddles[dev] = static_cast<const double2*>(ptr);
   hipError_t e = sigma_prepare();
   if (e != hipSuccess) return fail(KB_ERR_HIP, "sunset: transform pass set-up failed: %s", hipGetErrorString(e));
   g_ready[dev] = true;
   return KB_OK;
 }
 
-// the three plane passes over `nrows` rows; ws holds the twiddles and the rows
+// the passes over `nrows` rows
 int run_sunset(const kb_params* p, int nrows, const double* F, const double* rho, double* SigF, double* Sigr,
                char* ws, hipStream_t st) {
   const int n = p->Nx;
-  Twiddles tw{};
-  fft_twiddles(n, tw.w);
-  double2* dtw = reinterpret_cast<double2*>(ws);
-  hipLaunchKernelGGL(put_twiddles, dim3(1), dim3(NX_MAX), 0, st, tw, dtw, n);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return fail(KB_ERR_HIP, "sunset: twiddle launch failed: %s", hipGetErrorString(e));
   SigmaArgs a{};
-  a.W = reinterpret_cast<double2*>(ws + WS_TWIDDLE_BYTES);
-  a.tw = dtw;
+  a.W = reinterpret_cast<double2*>(ws + WS_HEAD_BYTES);
+  a.tw = g_twiddles[p->device] + twiddle_start(n);
   plan_fft(a.plan, n);
   a.n = a.nx = n;
   a.ny = p->sdim >= 2 ? n : 1;
@@ -160,8 +155,8 @@ int run_sunset(const kb_params* p, int nrows, const double* F, const double* rho
   a.Sigrout = Sigr;
   a.rows = nrows;
   a.classical = p->pexp == KB_PEXP_LAMBDA_NLO_CLASSICAL;
-  e = launch_sigma_stage(a, SG_PLAIN, nrows, st);
-  if (e != hipSuccess) return fail(KB_ERR_HIP, "sunset: plane kernel launch failed: %s", hipGetErrorString(e));
+  const hipError_t e = launch_sigma_stage(a, SG_PLAIN, nrows, st);
+  if (e != hipSuccess) return fail(KB_ERR_HIP, "sunset: transform launch failed: %s", hipGetErrorString(e));
   return KB_OK;
 }
 
