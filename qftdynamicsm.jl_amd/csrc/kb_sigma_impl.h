@@ -45,7 +45,7 @@
 // KIND_LAST reads the other half of a line from the reflected one and writes
 // both.
 //
-// Transforms.  n is cut into the fewest radices of 2 .. 11 and 13 (two up to
+// Transforms.  n is cut into the fewest radices of 2 .. 11, 13, 17, 19 and 23 (two up to
 // 100 or more; larger primes are a stage of their own), and one butterfly
 // lives in one thread's registers.  Where a line is transformed forth and
 // back, the last forward stage, the pointwise step and the first inverse stage
@@ -117,6 +117,35 @@ struct OddTable<13> {
                                   -0.35460488704253562597, -0.74851074817110109863, -0.97094181742605202716};
   static constexpr double s[7] = {0.0, 0.46472317204376854566, 0.82298386589365639458, 0.9927088740980539928,
                                   0.93501624268541482344, 0.66312265824079520238, 0.23931566428755776715};
+};
+template <>
+struct OddTable<17> {
+  static constexpr double c[9] = {1.0, 0.93247222940435580457, 0.73900891722065911592, 0.4457383557765382674,
+                                  0.09226835946330199524, -0.27366299007208286354, -0.60263463637925638918,
+                                  -0.85021713572961415213, -0.98297309968390177828};
+  static constexpr double s[9] = {0.0, 0.36124166618715294874, 0.67369564364655721171, 0.89516329135506232207,
+                                  0.99573417629503452187, 0.96182564317281907041, 0.79801722728023950333,
+                                  0.52643216287735580024, 0.18374951781657033157};
+};
+template <>
+struct OddTable<19> {
+  static constexpr double c[10] = {1.0, 0.94581724170063467902, 0.78914050939639359922, 0.54694815812242687471,
+                                  0.24548548714079914892, -0.0825793454723323246, -0.40169542465296945752,
+                                  -0.67728157162574107476, -0.87947375120648907139, -0.9863613034027223736};
+  static constexpr double s[10] = {0.0, 0.32469946920468348741, 0.61421271268966781744, 0.83716647826252857481,
+                                  0.96940026593933041674, 0.99658449300666984982, 0.91577332665505743992,
+                                  0.73572391067313162477, 0.47594739303707354443, 0.16459459028073389414};
+};
+template <>
+struct OddTable<23> {
+  static constexpr double c[12] = {1.0, 0.96291728734779929502, 0.85441940454648855255, 0.68255314321865408287,
+                                  0.46006503773115212604, 0.20345601305263378988, -0.068242413364670975921,
+                                  -0.33487961217098615196, -0.57668032211486714125, -0.77571129070441980704,
+                                  -0.91721130150545301784, -0.99068594603633075234};
+  static constexpr double s[12] = {0.0, 0.26979677115702427125, 0.51958395003543357813, 0.73083596427812410165,
+                                  0.88788521840237523498, 0.97908408768232287563, 0.99766876919053919845,
+                                  0.94226092211882049562, 0.81696989301044201697, 0.63108794432605278937,
+                                  0.398401089846241458, 0.13616664909624659076};
 };
 
 template <int R>
@@ -244,7 +273,7 @@ __device__ __forceinline__ void dft(double2 (&v)[R]) {
     v[2] = csub(a0, b0);
     v[1] = cadd(a1, b1);
     v[3] = csub(a1, b1);
-  } else if constexpr (R == 3 || R == 5 || R == 7 || R == 11 || R == 13) {
+  } else if constexpr (R == 3 || R == 5 || R == 7 || R == 11 || R == 13 || R == 17 || R == 19 || R == 23) {
     dft_odd<R>(v);
   } else if constexpr (R == 6) {
     dft_coprime<2, 3>(v);
@@ -430,8 +459,8 @@ constexpr int most(int a, int b) { return a > b ? a : b; }
 constexpr int held(int R) { return R == 1 ? 8 : most(1, 10 / R); }
 constexpr int DIRECT_PAIRS = 4, DIRECT_HELD = 2;  // output pairs per item of a prime stage, items per thread
 
-constexpr int RADICES[] = {13, 11, 10, 9, 8, 7, 6, 5, 4, 3, 2};
-constexpr bool is_direct(int R) { return R > 13; }
+constexpr int RADICES[] = {23, 19, 17, 13, 11, 10, 9, 8, 7, 6, 5, 4, 3, 2};
+constexpr bool is_direct(int R) { return R > 23; }
 constexpr size_t LDS_MAX = 160 * 1024;
 constexpr int LDS_VALUES = (int)(LDS_MAX / sizeof(double2));
 
@@ -443,16 +472,29 @@ constexpr int odd(int n) { return n | 1; }  // LDS stride of a line: neighbourin
 // How a pass knows its plan: a length NT > 0 is compiled in (whole rows up to
 // 26^3, planes at multiples of 8 up to 64, lines at powers of two: with every
 // index known a pass takes about two thirds of the time, 1024^1 N_mem = 200
-// 12.3 against 18.1 us); PLAN_SMALL runs any plan of radices up to 8 and
-// PLAN_ANY every plan.
-enum { PLAN_SMALL = 0, PLAN_ANY = -1 };
-constexpr int SMALL_RADIX = 8;
+// 12.3 against 18.1 us); PLAN_SMALL runs any plan of radices up to 8, PLAN_ANY
+// any without 17, 19 and 23, PLAN_WIDE every plan.
+enum { PLAN_SMALL = 0, PLAN_ANY = -1, PLAN_WIDE = -2 };
+constexpr int SMALL_RADIX = 8, ANY_RADIX = 13;
 // Waves per SIMD that the registers are cut for.  Six (80 registers) keep the
 // memory busy where four (the passes' natural 100) leave it waiting: 48^3 x
 // 100 rows 190 against 173 us; with the radices 9, 10 and the prime stages
 // the code would spill (47^3 x 24: 160 -> 195 us), so those plans have four.
 // A whole row has a CU to itself, or nearly, and 16 waves.
-constexpr int plan_waves(int kind, int nt) { return nt == PLAN_ANY || kind == KIND_WHOLE ? 4 : 6; }
+// The butterflies of 17, 19 and 23 need up to 230 registers: two waves, in
+// workgroups of up to 512 (as prime stages, whose outputs are shared out in
+// pairs, 17^3 N_mem = 100 took 55 us against 20, 34^3 N_mem = 60 over 200
+// against 116; of 29 they would spill).
+constexpr bool wide(const FFTPlan& pl) {
+  for (int i = 0; i < pl.nf; ++i)
+    if (pl.fac[i] > ANY_RADIX && !is_direct(pl.fac[i])) return true;
+  return false;
+}
+constexpr bool plan_wide(int nt);
+constexpr int plan_waves(int kind, int nt) {
+  return plan_wide(nt) ? 2 : nt == PLAN_ANY || kind == KIND_WHOLE ? 4 : 6;
+}
+constexpr int plan_threads(bool wide) { return wide ? 512 : 1024; }
 
 // the fewest radices with product m, descending; of those the smallest largest one
 constexpr void best_radices(int m, int maxR, int depth, int* cur, int* best, int& nbest) {
@@ -475,17 +517,17 @@ constexpr FFTPlan make_plan(int n) {
   FFTPlan pl{};
   pl.n = n;
   int m = n, primes[FFT_MAXF] = {}, np = 0;
-  for (int f : {2, 3, 5, 7, 11, 13})
+  for (int f : {2, 3, 5, 7, 11, 13, 17, 19, 23})
     while (m % f == 0) m /= f;
   const int smooth = n / m;
-  for (int f = 17; m > 1; f += 2)
+  for (int f = 29; m > 1; f += 2)
     while (m % f == 0) {
       primes[np++] = f;
       m /= f;
     }
   int cur[8] = {}, best[8] = {}, nbest = -1;
   if (smooth > 1) {
-    best_radices(smooth, 16, 0, cur, best, nbest);
+    best_radices(smooth, 23, 0, cur, best, nbest);
     for (int i = nbest - 1; i >= 0; --i) pl.fac[pl.nf++] = best[i];
   } else {
     pl.fac[pl.nf++] = 1;  // a prime stage does not read W
@@ -493,6 +535,8 @@ constexpr FFTPlan make_plan(int n) {
   for (int i = 0; i < np; ++i) pl.fac[pl.nf++] = primes[i];
   return pl;
 }
+
+constexpr bool plan_wide(int nt) { return nt > 0 ? wide(make_plan(nt)) : nt == PLAN_WIDE; }
 
 // The stages of one pass for workgroups of `threads`: a stage whose
 // butterflies they do not hold at once runs in chunks of lines.
@@ -576,7 +620,7 @@ constexpr int pass_threads(const FFTPlan& pl, int elements, int want, int fewest
     const int h = is_direct(R) ? DIRECT_HELD : held(R);
     per = most(per, (items + h - 1) / h);
   }
-  return (least(1024, most(per, least(most(want, elements / 16), elements / fewest))) + 63) / 64 * 64;
+  return (least(plan_threads(wide(pl)), most(per, least(most(want, elements / 16), elements / fewest))) + 63) / 64 * 64;
 }
 
 // lines per workgroup of a pass on batches: some 1536 values, and what LDS holds
@@ -591,10 +635,8 @@ constexpr int batch(int n, int limit) {
 constexpr bool planes_fit(int n) { return n <= 64; }
 // whole rows: the half space, and four lines that are their own reflection
 constexpr int whole_values(int n) { return n * odd(n) * (n / 2 + 1) + 4 * n; }
-// (a prime stage has too few outputs to give to so many threads: 23^3 N_mem =
-// 100 takes 119 us so, 72 in three passes)
 constexpr bool whole_fits(int n) {
-  return n >= 2 && whole_values(n) + n <= LDS_VALUES && !is_direct(make_plan(n).fac[make_plan(n).nf - 1]);  // n <= 26
+  return n >= 2 && whole_values(n) + n <= LDS_VALUES;  // n <= 26
 }
 constexpr int WHOLE_MAX = 26;
 // Compiled lengths from here on go by three passes, which fill the chip, while
@@ -984,7 +1026,15 @@ __device__ __forceinline__ void any_stage(const Stage& s, const Box<MODE, KIND>&
     case 7: run_stage<7>(s, box); break;
     case 8: run_stage<8>(s, box); break;
     default:
-      if constexpr (CLASS == PLAN_ANY) {
+      if constexpr (CLASS == PLAN_WIDE) {
+        if (s.R == 17)
+          return run_stage<17>(s, box);
+        else if (s.R == 19)
+          return run_stage<19>(s, box);
+        else if (s.R == 23)
+          return run_stage<23>(s, box);
+      }
+      if constexpr (CLASS == PLAN_ANY || CLASS == PLAN_WIDE) {
         if (s.R == 9)
           run_stage<9>(s, box);
         else if (s.R == 10)
@@ -1037,7 +1087,7 @@ __device__ __forceinline__ Stage stage_at(int i) {
 }
 
 template <int MODE, int KIND, int NT>
-__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(plan_waves(KIND, NT)))) void sigma_pass(
+__global__ __launch_bounds__(plan_threads(plan_wide(NT))) __attribute__((amdgpu_waves_per_eu(plan_waves(KIND, NT)))) void sigma_pass(
     SigmaArgs a, std::conditional_t<(NT > 0), NoPlan, PassPlan> plan) {
   const PassPlan& pp = [&]() -> const PassPlan& {
     if constexpr (NT > 0)
@@ -1141,11 +1191,14 @@ hipError_t launch_compiled(const SigmaArgs& a, dim3 grid, hipStream_t st) {
 template <int MODE, int KIND>
 hipError_t launch_pass(const SigmaArgs& a, const PassPlan& pp, dim3 grid, hipStream_t st) {
   const size_t lds = sizeof(double2) * ((size_t)pp.elements + pp.n);
-  if (lds + sizeof(pp.st) > LDS_MAX || pp.threads > 1024 || pp.nstages > MAX_STAGES) return hipErrorInvalidConfiguration;
+  const bool is_wide = wide(a.plan);
+  if (lds + sizeof(pp.st) > LDS_MAX || pp.threads > (is_wide ? 512 : 1024) || pp.nstages > MAX_STAGES) return hipErrorInvalidConfiguration;
   bool small = true;
   for (int i = 0; i < pp.nstages; ++i) small = small && pp.st[i].R <= SMALL_RADIX;
   if (small)
     hipLaunchKernelGGL((sigma_pass<MODE, KIND, PLAN_SMALL>), grid, dim3(pp.threads), lds, st, a, pp);
+  else if (is_wide)
+    hipLaunchKernelGGL((sigma_pass<MODE, KIND, PLAN_WIDE>), grid, dim3(pp.threads), lds, st, a, pp);
   else
     hipLaunchKernelGGL((sigma_pass<MODE, KIND, PLAN_ANY>), grid, dim3(pp.threads), lds, st, a, pp);
   return hipGetLastError();
@@ -1236,6 +1289,7 @@ template <int MODE>
 hipError_t prepare_mode() {
   hipError_t e = prepare_class<MODE, PLAN_SMALL>();
   if (e == hipSuccess) e = prepare_class<MODE, PLAN_ANY>();
+  if (e == hipSuccess) e = prepare_class<MODE, PLAN_WIDE>();
   if (e == hipSuccess) e = prepare_lengths<MODE, KIND_ROW, ROW_MIN, ROW_MAX, 0>();
   if (e == hipSuccess) e = prepare_lengths<MODE, KIND_WHOLE, 2, WHOLE_MAX, 1>();
   if (e == hipSuccess) e = prepare_lengths<MODE, KIND_ALL, 8, 64, 8>();

@@ -30,7 +30,8 @@ def sunset(F, r, lam, ON):
 # (Nx, sdim, rows)
 FORMS = [(n, 1, 3) for n in (1, 2, 3, 8, 9, 11, 13, 17, 32, 47, 60, 64)]
 FORMS += [(n, 2, 3) for n in (1, 2, 5, 8, 13, 17, 26, 32, 45, 56, 61, 63, 64)]
-FORMS += [(n, 3, 3) for n in (1, 2, 3, 8, 9, 10, 11, 13, 15, 16, 17, 22, 24, 25, 26, 27, 32, 34, 39, 40, 47)]
+FORMS += [(n, 3, 3) for n in (1, 2, 3, 8, 9, 10, 11, 13, 15, 16, 17, 19, 22, 23, 24, 25, 26, 27, 29, 32, 34, 39, 40,
+                                46, 47, 57)]
 FORMS += [(24, 3, 95), (24, 3, 96), (16, 3, 600), (49, 3, 2), (56, 3, 2), (63, 3, 1), (64, 3, 1)]
 
 
@@ -56,7 +57,8 @@ def test_sunset_forms(Nx, sdim, rows):
 # past Nx = 64 (no kb_sunset there): the stage of a step, against the transforms
 # of the rows it read
 @pytest.mark.parametrize("Nx,sdim", [(100, 1), (128, 1), (251, 1), (500, 1), (1024, 1), (2000, 1),
-                                     (65, 2), (66, 2), (97, 2), (131, 2), (256, 2), (65, 3), (67, 3), (72, 3), (99, 3)])
+                                     (65, 2), (66, 2), (69, 2), (87, 2), (97, 2), (131, 2), (256, 2),
+                                     (65, 3), (67, 3), (72, 3), (76, 3), (99, 3)])
 def test_batched_passes(Nx, sdim):
     from qftkb import KBContext
     print(f"\n[case] stage {Nx}^{sdim}", flush=True)
