@@ -875,10 +875,7 @@ static int create_ctx(const kb_params* p, bool sym, kb_ctx** out) {
     // holds device addresses: filled in once the arena has one
     const size_t margs_off = used;
     with((void**)&c->margs_dev, nullptr, sizeof(MemintArgs));
-    if (sym || c->hstage_n == 2 * HSTAGE_MAX) place((void**)&c->modes, (size_t)6 * c->V * sizeof(double));
-    // staging: 4 lattices
     place((void**)&c->partial, (size_t)6 * meas_groups(c->N, c->NB) * sizeof(double));
-    place((void**)&c->vbuf, 4 * (size_t)c->V * sizeof(double));
     if ((rc = dmalloc(c, &c->arena, used))) return fail(rc);
     for (const Part& q : parts) *q.ptr = static_cast<char*>(c->arena) + q.off;
     c->items = c->items_r[1];
