@@ -808,9 +808,10 @@ static int create_ctx(const kb_params* p, bool sym, kb_ctx** out) {
   if (c->fft_tile != KB_FFT_ORBIT_PRODUCT && (rc = ensure_plane_workspace(c))) return fail(rc);
   c->hstage_n = std::max((size_t)6 * c->Vl, (size_t)4 * c->N);
   if (c->hstage_n > HSTAGE_MAX) c->hstage_n = 2 * HSTAGE_MAX;
-  // The small buffers live in one allocation: first those with initial
-  // values, copied from a host image in one transfer (a context of a small
-  // lattice spent most of its creation on some thirty allocations and copies)
+  // The buffers that do not grow with the window's square live in one
+  // allocation: first those with initial values, copied from a host image in
+  // one transfer (a context of a small lattice spent most of its creation on
+  // some thirty allocations and copies)
   {
     struct Part {
       void** ptr;
@@ -876,6 +877,8 @@ static int create_ctx(const kb_params* p, bool sym, kb_ctx** out) {
     const size_t margs_off = used;
     with((void**)&c->margs_dev, nullptr, sizeof(MemintArgs));
     place((void**)&c->partial, (size_t)6 * meas_groups(c->N, c->NB) * sizeof(double));
+    place((void**)&c->modes, (size_t)6 * c->V * sizeof(double));
+    place((void**)&c->vbuf, (size_t)4 * c->V * sizeof(double));
     if ((rc = dmalloc(c, &c->arena, used))) return fail(rc);
     for (const Part& q : parts) *q.ptr = static_cast<char*>(c->arena) + q.off;
     c->items = c->items_r[1];
@@ -887,10 +890,6 @@ static int create_ctx(const kb_params* p, bool sym, kb_ctx** out) {
       hipSuccess)
     return fail(KB_ERR_OOM);
   c->hdata = c->hstage + HSTAGE_SCALARS;
-  if ((rc = dmalloc(c, (void**)&c->modes, (size_t)6 * c->V * sizeof(double)))) return fail(rc);
-  // staging: 4 lattices, or the 4 site-1 history vectors of kb_measure_history
-  const size_t vlen = (size_t)(c->V > c->N ? c->V : c->N);
-  if ((rc = dmalloc(c, (void**)&c->vbuf, 4 * vlen * sizeof(double)))) return fail(rc);
   if (sigma_prepare() != hipSuccess) {
     seterr(c, KB_ERR_ARG, "self-energy passes: LDS attribute rejected");
     return fail(KB_ERR_ARG);

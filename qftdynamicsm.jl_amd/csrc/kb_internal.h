@@ -51,8 +51,8 @@ struct kb_ctx {
   bool in_ensemble = false;
   double initmass = 0.0;      // set by kb_init_particles
   bool init_particles = false;
-  // device memory; the small buffers (from m2 on, the maps above and the
-  // launch tables below) share one allocation
+  // device memory; kL2, the buffers from m2 on, the maps above and the launch
+  // tables below share one allocation, the only one of theirs to free
   void* arena = nullptr;
   double* H = nullptr;     // history
   double* S = nullptr;     // self-energy ring
