@@ -64,8 +64,9 @@ struct kb_ctx {
   double* modes = nullptr; // 6 x V measurement outputs
   double* vbuf = nullptr;  // 4 x V staging
   // pinned host memory through which results leave the device: the scalars
-  // of a measurement, then hstage_n doubles of lattices (all six of a
-  // measurement where they fit HSTAGE_MAX, else two buffers of half that)
+  // of a measurement, then hstage_n doubles of stored sites (all six arrays of
+  // a measurement where six lattices fit HSTAGE_MAX, else two buffers of half
+  // that)
   double* hstage = nullptr;
   double* hdata = nullptr;
   size_t hstage_n = 0;

@@ -241,7 +241,6 @@ extern const MemintVariant kMemintVariants[NMEMINT_VARIANTS];
 constexpr int MEMINT_ROW_CHOICES[3] = {32, 64, 128};  // item tables kept per context
 __global__ void measure_kernel(MeasArgs a);
 __global__ void measure_finish(MeasArgs a, int groups);
-__global__ void expand_kernel(const double* src, int V, const int* smap, int Vl, int narr, double* dst);
 __global__ void history_kernel(const double* H, const double* S, long NP, int N, int tmin, int t, double* out);
 __global__ void gather_pair(const double* H, long NP, int V, long pair, int comp, double sign, double* out);
 __global__ void scatter_pair(double* H, long NP, int V, long pair, int comp, double sign, const double* in);

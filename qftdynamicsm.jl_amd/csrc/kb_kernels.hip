@@ -964,15 +964,6 @@ __global__ __launch_bounds__(MEAS_THREADS) void measure_finish(MeasArgs a, int G
   if (tid == 6) a.sums[6] = a.m2[0];
 }
 
-// narr arrays of V stored sites to the whole lattice (orbit storage)
-__global__ void expand_kernel(const double* __restrict__ src, int V, const int* __restrict__ smap, int Vl, int narr,
-                              double* __restrict__ dst) {
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= Vl) return;
-  const int r = smap[s];
-  for (int k = 0; k < narr; ++k) dst[(size_t)k * Vl + s] = src[(size_t)k * V + r];
-}
-
 // site-1 history (Measurement.jl:90-96); q = 0 .. t-tmin-1
 __global__ void history_kernel(const double* __restrict__ H, const double* __restrict__ S, long NP, int N,
                                int tmin, int t, double* __restrict__ out) {
