@@ -1320,6 +1320,8 @@ int adj_record(kb_ctx* c, int checkpoint_every, int max_steps, int host_windows)
                               (int)apply_lds());
     if (e != hipSuccess)
       return seterr(c, KB_ERR_ARG, "adjoint: %zu bytes of LDS rejected: %s", lds, hipGetErrorString(e));
+    int rc;
+    if (sunset_expansion(c->p.pexp) && (rc = prepare_sigma(c, SG_SUNSET_ADJ))) return rc;
   }
   HIPCHK(c, hipStreamSynchronize(c->stream));
   adj_free(c);

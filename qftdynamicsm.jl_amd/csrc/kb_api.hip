@@ -614,13 +614,22 @@ int dmalloc(kb_ctx* c, void** ptr, size_t bytes) {
   return KB_OK;
 }
 
+int prepare_sigma(kb_ctx* c, SigmaMode mode) {
+  const hipError_t e = sigma_prepare(mode, c->p.Nx, c->p.sdim, c->p.device);
+  if (e == hipSuccess) return KB_OK;
+  return seterr(c, KB_ERR_ARG, "self-energy passes: LDS attribute rejected: %s", hipGetErrorString(e));
+}
+
 // The transform passes' workspace: W holds the half space of each row between
 // the passes; Xn keeps the 1/N bubble pass's transforms for its chain pass.
-// Allocated when that form of the stage is first selected: LambdaLO and
-// contexts on the orbit products never hold them.
+// Allocated, and the passes prepared, when that form of the stage is first
+// selected: LambdaLO and contexts on the orbit products never hold them.
 int ensure_plane_workspace(kb_ctx* c) {
   if (!has_sigma(c)) return KB_OK;
   int rc;
+  if ((rc = prepare_sigma(c, c->p.pexp == KB_PEXP_NINVERSE_NLO ? SG_BUBBLE : SG_SUNSET)) ||
+      (c->p.pexp == KB_PEXP_NINVERSE_NLO && (rc = prepare_sigma(c, SG_CHAIN))))
+    return rc;
   const size_t rows = (size_t)c->N * c->Vl * sizeof(double2);
   const size_t wvals = sigma_workspace_values(c->p.Nx, c->p.sdim, c->N);
   if (wvals && !c->W && (rc = dmalloc(c, (void**)&c->W, wvals * sizeof(double2)))) return rc;
@@ -894,10 +903,6 @@ static int create_ctx(const kb_params* p, bool sym, kb_ctx** out) {
       hipSuccess)
     return fail(KB_ERR_OOM);
   c->hdata = c->hstage + HSTAGE_SCALARS;
-  if (sigma_prepare() != hipSuccess) {
-    seterr(c, KB_ERR_ARG, "self-energy passes: LDS attribute rejected");
-    return fail(KB_ERR_ARG);
-  }
   {
     // the attribute is per function, shared by every context: allow the
     // largest supported window, not this context's

@@ -164,6 +164,8 @@ int launch_sigma(kb_ctx* c, double2* X = nullptr, double* S_out = nullptr);
 // the plane kernels' workspace (W, and Xn for the 1/N passes), allocated
 // when a plane form is first selected; and whether it is missing
 int ensure_plane_workspace(kb_ctx* c);
+// sigma_prepare for the context's lattice and device (the current one)
+int prepare_sigma(kb_ctx* c, qftkb::SigmaMode mode);
 bool plane_workspace_missing(const kb_ctx* c);
 // Hartreeprefactor of the context's expansion (Initialization.jl:245-247)
 double hartree_prefactor(const kb_ctx* c);

@@ -264,7 +264,10 @@ void plan_fft(FFTPlan& pl, int n);
 size_t sigma_workspace_values(int Nx, int sdim, size_t rows);
 // the sizes whose stage serves orbit storage: Nx <= 64, and 1D up to 2048
 bool sigma_planes_supported(int Nx, int sdim);
-hipError_t sigma_prepare();  // LDS attribute of the passes
+// before a mode's first launch on lattices of Nx^sdim sites (Nx = 0: on any):
+// the LDS attributes of the passes they run and their code, once per device
+// (the current one)
+hipError_t sigma_prepare(SigmaMode mode, int Nx, int sdim, int device);
 // variant: index into kFFTThreads (threads per workgroup asked for)
 constexpr int NFFT_VARIANTS = 4;
 extern const int kFFTThreads[NFFT_VARIANTS];

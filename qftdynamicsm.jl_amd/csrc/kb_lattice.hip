@@ -127,7 +127,7 @@ int device_setup(int dev) {
   if (se != hipSuccess || !ptr)
     return fail(KB_ERR_HIP, "sunset: no device address for the twiddles: %s", hipGetErrorString(se));
   g_twiddles[dev] = static_cast<const double2*>(ptr);
-  hipError_t e = sigma_prepare();
+  hipError_t e = sigma_prepare(SG_PLAIN, 0, 0, dev);
   if (e != hipSuccess) return fail(KB_ERR_HIP, "sunset: transform pass set-up failed: %s", hipGetErrorString(e));
   g_ready[dev] = true;
   return KB_OK;

@@ -1,20 +1,80 @@
-// kb_sigma.hip -- self-energy stage (kb_sigma_impl.h): the sunset's passes and
-// what is common to the modes.
+// kb_sigma.hip -- self-energy stage (kb_sigma_impl.h): what is common to the
+// modes, and the choice of the form.
+#include <mutex>
+
 #include "kb_sigma_impl.h"
 
 namespace qftkb {
 
-KB_SIGMA_MODE(SG_SUNSET)
+namespace {
+
+constexpr int SIGMA_DEVICES = 64;  // (further ones are prepared at every call)
+constexpr int FORMS[] = {FORM_COMPILED, PLAN_SMALL, PLAN_ANY, PLAN_WIDE};
+constexpr int NFORMS = 4, NMODES = SG_PLAIN + 1;
+
+struct FormCode {
+  hipError_t (*launch)(const SigmaArgs&, int, int, hipStream_t);
+  hipError_t (*prepare)();
+};
+
+}  // namespace
+
+#define KB_FORM(MODE, FORM)                                                            \
+  template <>                                                                          \
+  hipError_t sigma_form<MODE, FORM>(const SigmaArgs&, int rows, int want, hipStream_t st); \
+  template <>                                                                          \
+  hipError_t sigma_form_prepare<MODE, FORM>();
+#define KB_MODE(MODE) \
+  KB_FORM(MODE, FORM_COMPILED) KB_FORM(MODE, PLAN_SMALL) KB_FORM(MODE, PLAN_ANY) KB_FORM(MODE, PLAN_WIDE)
+KB_MODE(SG_SUNSET)
+KB_MODE(SG_SUNSET_ADJ)
+KB_MODE(SG_BUBBLE)
+KB_MODE(SG_CHAIN)
+KB_MODE(SG_PLAIN)
+#undef KB_MODE
+#undef KB_FORM
+
+namespace {
+
+// (in the order of SigmaMode and of FORMS)
+#define KB_FORM(MODE, FORM) {sigma_form<MODE, FORM>, sigma_form_prepare<MODE, FORM>}
+#define KB_MODE(MODE) \
+  {KB_FORM(MODE, FORM_COMPILED), KB_FORM(MODE, PLAN_SMALL), KB_FORM(MODE, PLAN_ANY), KB_FORM(MODE, PLAN_WIDE)}
+const FormCode kForms[NMODES][NFORMS] = {KB_MODE(SG_SUNSET), KB_MODE(SG_SUNSET_ADJ), KB_MODE(SG_BUBBLE),
+                                         KB_MODE(SG_CHAIN), KB_MODE(SG_PLAIN)};
+#undef KB_MODE
+#undef KB_FORM
+
+int form_index(int form) {
+  int i = 0;
+  while (FORMS[i] != form) ++i;
+  return i;
+}
+
+}  // namespace
 
 void plan_fft(FFTPlan& pl, int n) { pl = make_plan(n); }
 
-hipError_t sigma_prepare() {
-  hipError_t e = sigma_prepare_mode<SG_SUNSET>();
-  if (e == hipSuccess) e = sigma_prepare_mode<SG_SUNSET_ADJ>();
-  if (e == hipSuccess) e = sigma_prepare_mode<SG_BUBBLE>();
-  if (e == hipSuccess) e = sigma_prepare_mode<SG_CHAIN>();
-  if (e == hipSuccess) e = sigma_prepare_mode<SG_PLAIN>();
-  return e;
+// A first call on a device also loads the form's code there (some 1.2 ms per
+// MB: all of it took 13 ms of a process's first kb_create), so only what a
+// lattice runs is prepared.
+hipError_t sigma_prepare(SigmaMode mode, int Nx, int sdim, int device) {
+  static std::mutex mu;
+  static bool ready[SIGMA_DEVICES][NMODES][NFORMS] = {};
+  bool used[NFORMS] = {};
+  if (Nx > 0) {
+    const FFTPlan pl = make_plan(Nx);
+    for (int rows : {1, SPREAD_ROWS}) used[form_index(stage_form(pl, sdim, rows))] = true;
+  }
+  std::lock_guard<std::mutex> lk(mu);
+  const bool known = device >= 0 && device < SIGMA_DEVICES;
+  for (int f = 0; f < NFORMS; ++f) {
+    if ((Nx > 0 && !used[f]) || (known && ready[device][mode][f])) continue;
+    const hipError_t e = kForms[mode][f].prepare();
+    if (e != hipSuccess) return e;
+    if (known) ready[device][mode][f] = true;
+  }
+  return hipSuccess;
 }
 
 // (3D rows that a workgroup holds whole do without; the workspace is part of
@@ -32,14 +92,8 @@ bool sigma_planes_supported(int Nx, int sdim) { return Nx >= 1 && Nx <= (sdim ==
 const int kFFTThreads[NFFT_VARIANTS] = {256, 128, 512, 1024};
 
 hipError_t launch_sigma_stage(const SigmaArgs& a, SigmaMode mode, int rows, hipStream_t st, int variant) {
-  const int want = kFFTThreads[variant];
-  switch (mode) {
-    case SG_SUNSET: return sigma_stage<SG_SUNSET>(a, rows, want, st);
-    case SG_SUNSET_ADJ: return sigma_stage<SG_SUNSET_ADJ>(a, rows, want, st);
-    case SG_BUBBLE: return sigma_stage<SG_BUBBLE>(a, rows, want, st);
-    case SG_CHAIN: return sigma_stage<SG_CHAIN>(a, rows, want, st);
-    default: return sigma_stage<SG_PLAIN>(a, rows, want, st);
-  }
+  const int form = stage_form(a.plan, a.ny == 1 ? 1 : a.nz == 1 ? 2 : 3, rows);
+  return kForms[mode][form_index(form)].launch(a, rows, kFFTThreads[variant], st);
 }
 
 }  // namespace qftkb

@@ -71,6 +71,7 @@
 #include <type_traits>
 
 #include "kb_kernels.h"
+#include "kb_twiddles.h"
 
 namespace qftkb {
 
@@ -1188,19 +1189,34 @@ hipError_t launch_compiled(const SigmaArgs& a, dim3 grid, hipStream_t st) {
   return hipGetLastError();
 }
 
-template <int MODE, int KIND>
+// the forms that the code of a mode comes in, each in an object file of its
+// own: FORM_COMPILED, the compiled lengths, and the classes of run-time plans
+constexpr int FORM_COMPILED = 1;
+
+constexpr int plan_class(const FFTPlan& pl) {
+  int top = 0;
+  for (int i = 0; i < pl.nf; ++i) top = most(top, pl.fac[i]);
+  return top <= SMALL_RADIX ? PLAN_SMALL : wide(pl) ? PLAN_WIDE : PLAN_ANY;
+}
+constexpr bool row_compiled(int n) { return n >= ROW_MIN && n <= ROW_MAX && (n & (n - 1)) == 0; }
+constexpr bool by_whole_rows(int n, int rows) {
+  return whole_fits(n) && (n % 8 || n < SPREAD_MIN || rows >= SPREAD_ROWS);
+}
+// the form of a stage over `rows` rows
+constexpr int stage_form(const FFTPlan& pl, int sdim, int rows) {
+  const int n = pl.n;
+  const bool compiled = sdim == 1 || n == 1 ? row_compiled(n)
+                                            : (sdim == 3 && by_whole_rows(n, rows)) || (planes_fit(n) && n % 8 == 0);
+  return compiled ? FORM_COMPILED : plan_class(pl);
+}
+
+template <int MODE, int KIND, int CLASS>
 hipError_t launch_pass(const SigmaArgs& a, const PassPlan& pp, dim3 grid, hipStream_t st) {
   const size_t lds = sizeof(double2) * ((size_t)pp.elements + pp.n);
-  const bool is_wide = wide(a.plan);
-  if (lds + sizeof(pp.st) > LDS_MAX || pp.threads > (is_wide ? 512 : 1024) || pp.nstages > MAX_STAGES) return hipErrorInvalidConfiguration;
-  bool small = true;
-  for (int i = 0; i < pp.nstages; ++i) small = small && pp.st[i].R <= SMALL_RADIX;
-  if (small)
-    hipLaunchKernelGGL((sigma_pass<MODE, KIND, PLAN_SMALL>), grid, dim3(pp.threads), lds, st, a, pp);
-  else if (is_wide)
-    hipLaunchKernelGGL((sigma_pass<MODE, KIND, PLAN_WIDE>), grid, dim3(pp.threads), lds, st, a, pp);
-  else
-    hipLaunchKernelGGL((sigma_pass<MODE, KIND, PLAN_ANY>), grid, dim3(pp.threads), lds, st, a, pp);
+  if (lds + sizeof(pp.st) > LDS_MAX || pp.threads > plan_threads(CLASS == PLAN_WIDE) || pp.nstages > MAX_STAGES ||
+      plan_class(a.plan) != CLASS)
+    return hipErrorInvalidConfiguration;
+  hipLaunchKernelGGL((sigma_pass<MODE, KIND, CLASS>), grid, dim3(pp.threads), lds, st, a, pp);
   return hipGetLastError();
 }
 
@@ -1217,45 +1233,52 @@ hipError_t launch_length(const SigmaArgs& a, int n, dim3 grid, hipStream_t st) {
     return hipErrorInvalidConfiguration;
 }
 
-// want: threads per workgroup asked for (plans that are not compiled)
+// the longest compiled line of a mode (SG_PLAIN has no lattice past TWIDDLE_MAX)
 template <int MODE>
-hipError_t launch_stage(const SigmaArgs& a, int rows, int want, hipStream_t st) {
-  const FFTPlan& pl = a.plan;
+constexpr int row_last = MODE == SG_PLAIN ? TWIDDLE_MAX : ROW_MAX;
+
+template <int MODE>
+hipError_t launch_compiled_stage(const SigmaArgs& a, int rows, hipStream_t st) {
   const int n = a.n;
-  if (a.ny == 1) {
-    if (n >= ROW_MIN && n <= ROW_MAX && (n & (n - 1)) == 0)
-      return launch_length<MODE, KIND_ROW, ROW_MIN, ROW_MAX, 0>(a, n, dim3(1, rows), st);
-    return launch_pass<MODE, KIND_ROW>(a, pass_plan(pl, KIND_ROW, false, want), dim3(1, rows), st);
-  }
-  const bool three = a.nz > 1, planes = planes_fit(n);
-  if (three && whole_fits(n) && (n % 8 || n < SPREAD_MIN || rows >= SPREAD_ROWS))
-    return launch_length<MODE, KIND_WHOLE, 2, WHOLE_MAX, 1>(a, n, dim3(1, rows), st);
-  if (planes && !three) {
-    if (n % 8 == 0) return launch_length<MODE, KIND_ALL, 8, 64, 8>(a, n, dim3(1, rows), st);
-    return launch_pass<MODE, KIND_ALL>(a, pass_plan(pl, KIND_ALL, false, want), dim3(1, rows), st);
-  }
+  if (a.ny == 1) return launch_length<MODE, KIND_ROW, ROW_MIN, row_last<MODE>, 0>(a, n, dim3(1, rows), st);
+  if (a.nz == 1) return launch_length<MODE, KIND_ALL, 8, 64, 8>(a, n, dim3(1, rows), st);
+  if (by_whole_rows(n, rows)) return launch_length<MODE, KIND_WHOLE, 2, WHOLE_MAX, 1>(a, n, dim3(1, rows), st);
+  const PassPlan last = pass_plan(a.plan, KIND_LAST, true, CT_WANT);
   const int nh = n / 2 + 1;
+  const dim3 gx(nh, rows), gl(last.tiles * nh, rows);
   hipError_t e;
-  if (planes && n % 8 == 0) {
-    const PassPlan last = pass_plan(pl, KIND_LAST, true, CT_WANT);
-    const dim3 gx(nh, rows), gl(last.tiles * nh, rows);
-    if ((e = launch_length<MODE, KIND_FWD, SPREAD_MIN, 64, 8>(a, n, gx, st)) != hipSuccess) return e;
-    if ((e = launch_length<MODE, KIND_LAST, SPREAD_MIN, 64, 8>(a, n, gl, st)) != hipSuccess) return e;
-    return launch_length<MODE, KIND_INV, SPREAD_MIN, 64, 8>(a, n, gx, st);
-  }
+  if ((e = launch_length<MODE, KIND_FWD, SPREAD_MIN, 64, 8>(a, n, gx, st)) != hipSuccess) return e;
+  if ((e = launch_length<MODE, KIND_LAST, SPREAD_MIN, 64, 8>(a, n, gl, st)) != hipSuccess) return e;
+  return launch_length<MODE, KIND_INV, SPREAD_MIN, 64, 8>(a, n, gx, st);
+}
+
+// want: threads per workgroup asked for
+template <int MODE, int CLASS>
+hipError_t launch_plan_stage(const SigmaArgs& a, int rows, int want, hipStream_t st) {
+  const FFTPlan& pl = a.plan;
+  const int n = a.n, nh = n / 2 + 1;
+  if (a.ny == 1)
+    return launch_pass<MODE, KIND_ROW, CLASS>(a, pass_plan(pl, KIND_ROW, false, want), dim3(1, rows), st);
+  const bool three = a.nz > 1, planes = planes_fit(n);
+  if (planes && !three)
+    return launch_pass<MODE, KIND_ALL, CLASS>(a, pass_plan(pl, KIND_ALL, false, want), dim3(1, rows), st);
   const PassPlan fwd = pass_plan(pl, KIND_FWD, three, want), mid = pass_plan(pl, KIND_MID, three, want);
   const PassPlan last = pass_plan(pl, KIND_LAST, three, want), inv = pass_plan(pl, KIND_INV, three, want);
   const dim3 gx(planes ? nh : (fwd.total + fwd.lines - 1) / fwd.lines, rows), gm(mid.tiles * nh, rows),
       gl(last.tiles * (three ? nh : 1), rows);
-  if ((e = launch_pass<MODE, KIND_FWD>(a, fwd, gx, st)) != hipSuccess) return e;
-  // (the pass between planes and last axis does not depend on the mode)
   const bool between = three && !planes;
-  if (between && (e = launch_pass<MODE == SG_PLAIN ? SG_PLAIN : SG_SUNSET, KIND_MID>(a, mid, gm, st)) != hipSuccess)
-    return e;
-  if ((e = launch_pass<MODE, KIND_LAST>(a, last, gl, st)) != hipSuccess) return e;
-  if (between && (e = launch_pass<MODE == SG_PLAIN ? SG_PLAIN : SG_SUNSET, KIND_MID>(a, mid, gm, st)) != hipSuccess)
-    return e;
-  return launch_pass<MODE, KIND_INV>(a, inv, gx, st);
+  auto middle = [&]() -> hipError_t {
+    if constexpr (MODE == SG_PLAIN)
+      return hipErrorInvalidConfiguration;  // (no lattice of that size)
+    else
+      return launch_pass<MODE, KIND_MID, CLASS>(a, mid, gm, st);
+  };
+  hipError_t e;
+  if ((e = launch_pass<MODE, KIND_FWD, CLASS>(a, fwd, gx, st)) != hipSuccess) return e;
+  if (between && (e = middle()) != hipSuccess) return e;
+  if ((e = launch_pass<MODE, KIND_LAST, CLASS>(a, last, gl, st)) != hipSuccess) return e;
+  if (between && (e = middle()) != hipSuccess) return e;
+  return launch_pass<MODE, KIND_INV, CLASS>(a, inv, gx, st);
 }
 
 // the dynamic LDS that the larger passes need, per kernel
@@ -1277,20 +1300,18 @@ hipError_t prepare_lengths() {
     return e;
 }
 template <int MODE, int CLASS>
-hipError_t prepare_class() {
+hipError_t prepare_plan_stage() {
   hipError_t e = prepare_pass<MODE, KIND_ROW, CLASS>();
   if (e == hipSuccess) e = prepare_pass<MODE, KIND_ALL, CLASS>();
   if (e == hipSuccess) e = prepare_pass<MODE, KIND_FWD, CLASS>();
-  if (e == hipSuccess) e = prepare_pass<MODE, KIND_MID, CLASS>();
+  if constexpr (MODE != SG_PLAIN)
+    if (e == hipSuccess) e = prepare_pass<MODE, KIND_MID, CLASS>();
   if (e == hipSuccess) e = prepare_pass<MODE, KIND_LAST, CLASS>();
   return e == hipSuccess ? prepare_pass<MODE, KIND_INV, CLASS>() : e;
 }
 template <int MODE>
-hipError_t prepare_mode() {
-  hipError_t e = prepare_class<MODE, PLAN_SMALL>();
-  if (e == hipSuccess) e = prepare_class<MODE, PLAN_ANY>();
-  if (e == hipSuccess) e = prepare_class<MODE, PLAN_WIDE>();
-  if (e == hipSuccess) e = prepare_lengths<MODE, KIND_ROW, ROW_MIN, ROW_MAX, 0>();
+hipError_t prepare_compiled_stage() {
+  hipError_t e = prepare_lengths<MODE, KIND_ROW, ROW_MIN, row_last<MODE>, 0>();
   if (e == hipSuccess) e = prepare_lengths<MODE, KIND_WHOLE, 2, WHOLE_MAX, 1>();
   if (e == hipSuccess) e = prepare_lengths<MODE, KIND_ALL, 8, 64, 8>();
   if (e == hipSuccess) e = prepare_lengths<MODE, KIND_FWD, SPREAD_MIN, 64, 8>();
@@ -1300,20 +1321,10 @@ hipError_t prepare_mode() {
 
 }  // namespace
 
-// the stage of one mode, each in a file of its own (they compile side by side)
-template <int MODE>
-hipError_t sigma_stage(const SigmaArgs& a, int rows, int want, hipStream_t st);
-template <int MODE>
-hipError_t sigma_prepare_mode();
-
-#define KB_SIGMA_MODE(MODE)                                                                       \
-  template <>                                                                                     \
-  hipError_t sigma_stage<MODE>(const SigmaArgs& a, int rows, int want, hipStream_t st) {          \
-    return launch_stage<MODE>(a, rows, want, st);                                                 \
-  }                                                                                               \
-  template <>                                                                                     \
-  hipError_t sigma_prepare_mode<MODE>() {                                                         \
-    return prepare_mode<MODE>();                                                                  \
-  }
+// the stage of one mode in one form, and its preparation (kb_sigma_pass.hip)
+template <int MODE, int FORM>
+hipError_t sigma_form(const SigmaArgs& a, int rows, int want, hipStream_t st);
+template <int MODE, int FORM>
+hipError_t sigma_form_prepare();
 
 }  // namespace qftkb
