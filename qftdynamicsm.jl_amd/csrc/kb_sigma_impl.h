@@ -289,38 +289,48 @@ __device__ __forceinline__ void dft(double2 (&v)[R]) {
 
 // ---------------------------------------------------------------------------
 // pointwise steps and outputs of the modes
+//
+// The fused multiply-adds of the pointwise steps are written out, and their
+// products are rounded: left to the compiler, they would be fused into the sums
+// of the inverse butterfly where it follows in the same block of code (compiled
+// lengths) and not elsewhere (run-time plans).  A row's values do not depend on
+// the form that computes it: a row of kb_sunset has the bits of a step's.
 // ---------------------------------------------------------------------------
 // (Fx (Fx^2 - qF rx^2), rx (Fx^2 - qr rx^2)): qF = 3/4, qr = 1/12 for the
 // quantum sunset (Evolution.jl:25-31), 0 for the classical one (:107-120)
 __device__ __forceinline__ double2 sunset(double2 z, int classical) {
+#pragma clang fp contract(off)
   const double qF = classical ? 0.0 : 0.75, qr = classical ? 0.0 : 1.0 / 12.0;
   const double Fx = z.x, rx = z.y;
   const double FF = Fx * Fx, rr = rx * rx;
-  return make_double2(Fx * (FF - qF * rr), rx * (FF - qr * rr));
+  return make_double2(Fx * fma(-qF, rr, FF), rx * fma(-qr, rr, FF));
 }
 
 // transpose of the sunset's Jacobian at (Fx, rx) applied to
 // (gF, gr) = (preF, preR) * (C SigF_bar, C Sigr_bar)
 __device__ __forceinline__ double2 sunset_adj(double2 cs, double2 x, double preF, double preR, int classical) {
+#pragma clang fp contract(off)
   const double a1 = classical ? 0.0 : 0.75, a2 = classical ? 0.0 : -1.5, a3 = classical ? 0.0 : 0.25;
   const double gF = preF * cs.x, gr = preR * cs.y;
   const double Fx = x.x, rx = x.y;
   const double FF = Fx * Fx, rr = rx * rx;
-  return make_double2(gF * (3.0 * FF - a1 * rr) + gr * (2.0 * rx * Fx), gF * (a2 * Fx * rx) + gr * (FF - a3 * rr));
+  return make_double2(fma(gF, fma(-a1, rr, 3.0 * FF), gr * (2.0 * rx * Fx)),
+                      fma(gF, a2 * Fx * rx, gr * fma(-a3, rr, FF)));
 }
 
 // the pointwise step of each mode; the sunset and bubble save (Fx, rx) in X when it is set
 template <int MODE>
 __device__ __forceinline__ double2 pointwise(const SigmaArgs& a, double2 z, size_t xi) {
+#pragma clang fp contract(off)
   if constexpr (MODE == SG_SUNSET_ADJ) {
     return sunset_adj(z, a.X[xi], a.preF, a.preR, a.classical);
   } else if constexpr (MODE == SG_BUBBLE) {
     if (a.X) a.X[xi] = z;
-    return make_double2(z.x * z.x - 0.25 * (z.y * z.y), z.x * z.y);
+    return make_double2(fma(z.x, z.x, -0.25 * (z.y * z.y)), z.x * z.y);
   } else if constexpr (MODE == SG_CHAIN) {
     const double2 x = a.X[xi];  // (Fx, rx) of (t-1, t')
     const double IFx = a.ivol * z.x, Irx = a.ivol * z.y;
-    return make_double2(x.x * IFx - 0.25 * (x.y * Irx), x.x * Irx + x.y * IFx);
+    return make_double2(fma(x.x, IFx, -0.25 * (x.y * Irx)), fma(x.x, Irx, x.y * IFx));
   } else {
     if (a.X) a.X[xi] = z;
     return sunset(z, a.classical);
