@@ -32,7 +32,7 @@
 //   1D: one pass, KIND_ROW, a line per workgroup;
 //   2D, Nx <= 64: one pass, KIND_ALL, a plane per workgroup;
 //   3D, Nx <= 26: one pass, KIND_WHOLE, a whole row (its half space) per
-//       workgroup; see SPREAD_MIN for 24^3 with few rows;
+//       workgroup; see SPREAD_MIN for 24^3 to 26^3 with few rows;
 //   3D, Nx <= 64: KIND_FWD gathers plane z and its reflection -z and
 //       transforms x and y; KIND_LAST transforms z, applies the pointwise
 //       step and transforms back, on tiles of x; KIND_INV transforms y and x
@@ -650,13 +650,16 @@ constexpr bool whole_fits(int n) {
   return n >= 2 && whole_values(n) + n <= LDS_VALUES;  // n <= 26
 }
 constexpr int WHOLE_MAX = 26;
-// Compiled lengths from here on go by three passes, which fill the chip, while
-// there are few rows: a whole row keeps one CU busy for 33 us at 24^3, three
-// passes take 21 us for 8 rows, 26 for 50 and 40 for 150 (at 16^3 the two take
-// 16.5 us both for 8 rows, 17 and 19 for 64; at lengths that have no compiled
-// passes whole rows win from the first row on).
+// From here on rows go by three passes, which fill the chip, while there are
+// few of them: a whole row keeps one CU busy for 33 us at 24^3, three compiled
+// passes take 14 us for 1 row, 18 for 24 and 31 for 96, as long as whole rows
+// (at 16^3 the two take 16.5 us both for 8 rows, 17 and 19 for 64).  Lengths
+// that have no compiled passes change over earlier: 25^3 22 against 29 us for 1
+// row, 28 against 30 for 32, 32 against 31 for 48; 26^3 32 against 42, 38
+// against 44, 42 against 45.  (Below 24 whole rows win there from the first
+// row on: 22^3 28 against 32 us, 20^3 18 against 27.)
 constexpr int ROW_MIN = 8, ROW_MAX = 1024;  // compiled lines: powers of two
-constexpr int SPREAD_MIN = 24, SPREAD_ROWS = 96;
+constexpr int SPREAD_MIN = 24, SPREAD_ROWS = 96, SPREAD_PLAN_ROWS = 40;
 // lines along z that stand for themselves and their reflection (-x, -y)
 constexpr int whole_zlines(int n) { return (n % 2 ? 1 : 2) * (n / 2 + 1) + (n - 1) / 2 * n; }
 
@@ -1210,7 +1213,7 @@ constexpr int plan_class(const FFTPlan& pl) {
 }
 constexpr bool row_compiled(int n) { return n >= ROW_MIN && n <= ROW_MAX && (n & (n - 1)) == 0; }
 constexpr bool by_whole_rows(int n, int rows) {
-  return whole_fits(n) && (n % 8 || n < SPREAD_MIN || rows >= SPREAD_ROWS);
+  return whole_fits(n) && (n < SPREAD_MIN || rows >= (n % 8 ? SPREAD_PLAN_ROWS : SPREAD_ROWS));
 }
 // the form of a stage over `rows` rows
 constexpr int stage_form(const FFTPlan& pl, int sdim, int rows) {

@@ -1,0 +1,75 @@
+"""A few rows of the largest lattices that a workgroup holds whole go by three
+passes: the values against numpy's FFT on both sides of the change (1e-12 of
+the largest value: some 10 log2(V) roundings of 1.1e-16), the bits of a step
+on both sides of it, and one row of 25^3 taking no longer than one of 27^3."""
+import time
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+class Rows:
+    def __init__(self, Nx, F, r):
+        from hipmem import DeviceArray
+        from qftkb._abi import sunset_workspace_bytes
+        self.Nx, self.rows = Nx, len(F)
+        self.F, self.r = DeviceArray.from_host(F), DeviceArray.from_host(r)
+        self.out = [DeviceArray(F.size) for _ in range(2)]
+        self.nb = sunset_workspace_bytes(Nx, 3, self.rows)
+        self.ws = DeviceArray(self.nb, np.uint8)
+
+    def run(self):
+        from qftkb._abi import sunset
+        sunset(self.Nx, 3, 1.7, 3, self.rows, self.F.ptr, self.r.ptr, self.out[0].ptr, self.out[1].ptr, self.ws.ptr,
+               self.nb)
+        return self
+
+    def host(self):
+        return [o.host().reshape(self.rows, -1) for o in self.out]
+
+
+def data(Nx, rows):
+    return np.random.default_rng(Nx).standard_normal((2, rows, Nx ** 3))
+
+
+@pytest.mark.parametrize("Nx", [24, 25, 26])
+def test_few_rows_match_many(Nx):
+    many = 97
+    F, r = data(Nx, many)
+    print(f"\n[case] few rows {Nx}^3", flush=True)
+    want = Rows(Nx, F, r).run().host()
+    sh = (Nx,) * 3
+    ivol = 1.0 / Nx ** 3
+    pre = -1.7 ** 2 * 5.0 / 9.0 * ivol ** 3
+    for q in (0, many - 1):
+        Fx, rx = np.fft.fftn(F[q].reshape(sh)).real, np.fft.fftn(r[q].reshape(sh)).real
+        SF = pre / 18.0 * np.fft.fftn(Fx * (Fx ** 2 - 0.75 * rx ** 2)).real.reshape(-1)
+        SR = pre / 6.0 * np.fft.fftn(rx * (Fx ** 2 - rx ** 2 / 12.0)).real.reshape(-1)
+        for got, ref in zip(want, (SF, SR)):
+            assert np.max(np.abs(got[q] - ref)) <= 1e-12 * np.max(np.abs(ref)), q
+    for rows in (1, 39, 40, 95, 96):
+        for got, ref in zip(Rows(Nx, F[:rows], r[:rows]).run().host(), want):
+            assert np.array_equal(got, ref[:rows]), rows
+
+
+def test_one_row_of_25_takes_no_longer_than_one_of_27():
+    from hipmem import synchronize
+    sets = [Rows(n, *data(n, 1)) for n in (25, 27)]
+    ratios = []
+    for _ in range(6):
+        best = []
+        for s in sets:
+            times = []
+            for _ in range(6):
+                synchronize()
+                t = time.perf_counter()
+                for _ in range(40):
+                    s.run()
+                synchronize()
+                times.append(time.perf_counter() - t)
+            best.append(min(times))
+        ratios.append(best[0] / best[1])
+    print(f"\n[case] one row of 25^3 over one of 27^3: {min(ratios):.2f}", flush=True)
+    assert min(ratios) <= 1.0  # (whole in one workgroup: 1.1)
