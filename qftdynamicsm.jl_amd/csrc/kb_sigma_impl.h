@@ -468,7 +468,14 @@ constexpr int least(int a, int b) { return a < b ? a : b; }
 constexpr int most(int a, int b) { return a > b ? a : b; }
 // butterflies of radix R that a thread's registers hold
 constexpr int held(int R) { return R == 1 ? 8 : most(1, 10 / R); }
-constexpr int DIRECT_PAIRS = 4, DIRECT_HELD = 2;  // output pairs per item of a prime stage, items per thread
+// Prime stages: output pairs per item, and items per thread.  A line alone in
+// its workgroup has an item for each pair: it has threads to spare, and a
+// quarter of them each with four pairs take twice the time (a step's stage and
+// the rest, N_mem = 8, us: 61^1 32 against 20, 251^1 80 against 37, 2039^1 501
+// against 352; kb_sunset of 300 rows of 61^1 27 against 11).
+constexpr int DIRECT_PAIRS = 4, DIRECT_HELD = 2;
+constexpr int direct_pairs(int kind) { return kind == KIND_ROW ? 1 : DIRECT_PAIRS; }
+constexpr int direct_groups(int kind, int R) { return ((R - 1) / 2 + direct_pairs(kind) - 1) / direct_pairs(kind); }
 
 constexpr int RADICES[] = {23, 19, 17, 13, 11, 10, 9, 8, 7, 6, 5, 4, 3, 2};
 constexpr bool is_direct(int R) { return R > 23; }
@@ -554,8 +561,9 @@ constexpr bool plan_wide(int nt) { return nt > 0 ? wide(make_plan(nt)) : nt == P
 struct Builder {
   PassPlan pp{};
   FFTPlan pl{};
+  int kind;
 
-  constexpr Builder(const FFTPlan& p, int lines, int elements, int threads) : pl(p) {
+  constexpr Builder(int k, const FFTPlan& p, int lines, int elements, int threads) : pl(p), kind(k) {
     pp.n = p.n;
     pp.threads = threads;
     pp.lines = lines;
@@ -564,9 +572,9 @@ struct Builder {
     pp.mgn = magic(p.n);
   }
   constexpr void add(int R, int Ns, int lines, int ls, int es, int flags) {
+    if (R == 1 && !(flags & (ST_SRC | ST_SNK | ST_POINT))) return;  // (needed at W only)
     const int m = pp.n / R;
-    const int groups = is_direct(R) ? ((R - 1) / 2 + DIRECT_PAIRS - 1) / DIRECT_PAIRS : 1;
-    const int per = m * groups;  // items of a line
+    const int per = m * (is_direct(R) ? direct_groups(kind, R) : 1);  // items of a line
     const int room = most(1, pp.threads * (is_direct(R) ? DIRECT_HELD : held(R)) / per);
     const int chunks = (lines + room - 1) / room, chunk = (lines + chunks - 1) / chunks;
     for (int first = 0; first < lines; first += chunk) {
@@ -623,11 +631,11 @@ struct Builder {
 // would not be held.  Passes whose rows have a CU to themselves take 2 or 4
 // (12^3 N_mem = 100 13.4 us with 2, 20 with 8; 16^3 N_mem = 202 18.3 with 4,
 // 20.8 with 8, and 2 costs 16^3 N_mem = 600 45 against 37).
-constexpr int pass_threads(const FFTPlan& pl, int elements, int want, int fewest = 8) {
+constexpr int pass_threads(int kind, const FFTPlan& pl, int elements, int want, int fewest = 8) {
   int per = 64;
   for (int i = 0; i < pl.nf; ++i) {
     const int R = pl.fac[i], m = pl.n / R;
-    const int items = is_direct(R) ? m * (((R - 1) / 2 + DIRECT_PAIRS - 1) / DIRECT_PAIRS) : m;
+    const int items = is_direct(R) ? m * direct_groups(kind, R) : m;
     const int h = is_direct(R) ? DIRECT_HELD : held(R);
     per = most(per, (items + h - 1) / h);
   }
@@ -669,7 +677,7 @@ constexpr PassPlan pass_plan(const FFTPlan& pl, int kind, bool three, int want) 
   const int nh = n / 2 + 1, xrows = three ? n * nh : nh;  // x rows of the half space
   if (kind == KIND_WHOLE) {
     const int ps = ls * n;
-    Builder b(pl, xrows, whole_values(n), pass_threads(pl, n * n * nh, 1024, n < 16 ? 2 : 4));
+    Builder b(kind, pl, xrows, whole_values(n), pass_threads(kind, pl, n * n * nh, 1024, n < 16 ? 2 : 4));
     b.pp.total = xrows;
     b.forward(xrows, ls, 1, 0);
     b.forward(n * nh, 1, ls, ST_Y);
@@ -679,7 +687,7 @@ constexpr PassPlan pass_plan(const FFTPlan& pl, int kind, bool three, int want) 
     return b.pp;
   }
   if (kind == KIND_ROW) {  // a line: two values per thread
-    Builder b(pl, 1, ls, pass_threads(pl, n, 1024, 2));
+    Builder b(kind, pl, 1, ls, pass_threads(kind, pl, n, 1024, 2));
     b.pp.total = 1;
     b.round_trip(1, ls, 1, 0);
     return b.pp;
@@ -687,7 +695,7 @@ constexpr PassPlan pass_plan(const FFTPlan& pl, int kind, bool three, int want) 
   const bool planes = planes_fit(n);
   if (kind == KIND_LAST || kind == KIND_MID) {
     const int xt = batch(n, n);
-    Builder b(pl, xt, xt * ls, pass_threads(pl, xt * n, want));
+    Builder b(kind, pl, xt, xt * ls, pass_threads(kind, pl, xt * n, want));
     b.pp.tiles = (n + xt - 1) / xt;
     if (kind == KIND_MID)
       b.forward(xt, ls, 1, 0, ST_SRC, ST_SNK);
@@ -696,7 +704,7 @@ constexpr PassPlan pass_plan(const FFTPlan& pl, int kind, bool three, int want) 
     return b.pp;
   }
   const int xr = planes ? n : batch(n, xrows);
-  Builder b(pl, xr, xr * ls, pass_threads(pl, xr * n, want, kind == KIND_ALL && n <= 32 ? 2 : 8));
+  Builder b(kind, pl, xr, xr * ls, pass_threads(kind, pl, xr * n, want, kind == KIND_ALL && n <= 32 ? 2 : 8));
   b.pp.total = kind == KIND_ALL ? n : xrows;
   if (kind == KIND_ALL) {
     b.forward(n, ls, 1, 0);
@@ -942,12 +950,12 @@ __device__ __forceinline__ void run_stage(const Stage& s, const Box<MODE, KIND>&
   if ((s.flags & ST_END) && !(s.flags & ST_SNK)) __syncthreads();
 }
 
-// a prime radix above 7, from LDS: an item forms DIRECT_PAIRS output pairs
-// q, R - q of one butterfly from the sums and differences of its inputs,
+// a prime radix above 23, from LDS: an item forms direct_pairs(KIND) output
+// pairs q, R - q of one butterfly from the sums and differences of its inputs,
 // X_q, X_{R-q} = A +- B (the odd DFT above with a table)
 template <int MODE, int KIND>
 __device__ __forceinline__ void run_direct(const Stage& s, const Box<MODE, KIND>& box) {
-  constexpr int G = DIRECT_PAIRS, U = DIRECT_HELD;
+  constexpr int G = direct_pairs(KIND), U = DIRECT_HELD;
   const int R = s.R, H = (R - 1) / 2;
   const int T = blockDim.x;
   const int step = s.Ns > 1 ? s.m / s.Ns : 0;
