@@ -30,7 +30,8 @@ constexpr DD dd_div(DD a, double d) {
   const DD r = dd_add(a, dd_neg(dd_mul({q, 0.0}, {d, 0.0})));
   return dd_sum(q, r.h / d);
 }
-struct TwiddleTable {
+// (aligned for the 16-byte loads of its pairs)
+struct alignas(16) TwiddleTable {
   double v[TWIDDLE_MAX * (TWIDDLE_MAX + 1)];  // (re, im) pairs
 };
 constexpr int twiddle_start(int n) { return n * (n - 1) / 2; }
