@@ -4,18 +4,16 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <atomic>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
-#include <exception>
 #include <new>
 #include <string>
-#include <thread>
 #include <vector>
 
 #include "../../include/qftkb.h"
+#include "kb_hostcopy.h"
 #include "kb_internal.h"
 #include "kb_twiddles.h"
 
@@ -464,19 +462,8 @@ int upload(kb_ctx* c, double* dst, const double* src, size_t n) {
 }
 
 // Device arrays of n doubles into caller arrays, through the context's pinned
-// memory.  What fits it goes in one copy.  Larger arrays go in halves of it,
-// the next half's copy running while HOST_COPY_THREADS threads write the
-// previous one out: the caller's fresh pages cost a single thread more time
-// than the copy.
-constexpr int HOST_COPY_THREADS = 6;
-
+// memory.  What fits it goes in one copy, larger arrays in halves of it.
 int download_many(kb_ctx* c, int narr, double* const* dst, const double* const* src, size_t n) {
-  struct Piece {
-    double* d;
-    const double* s;
-    size_t n;
-  };
-  const size_t half = c->hstage_n / 2;
   if (n * narr <= c->hstage_n) {
     for (int k = 0; k < narr; ++k)
       HIPCHK(c, hipMemcpyAsync(c->hdata + k * n, src[k], n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
@@ -484,60 +471,11 @@ int download_many(kb_ctx* c, int narr, double* const* dst, const double* const* 
     for (int k = 0; k < narr; ++k) std::memcpy(dst[k], c->hdata + k * n, n * sizeof(double));
     return KB_OK;
   }
-  std::vector<Piece> pieces;
-  for (int k = 0; k < narr; ++k)
-    for (size_t o = 0; o < n; o += half) pieces.push_back({dst[k] + o, src[k] + o, std::min(half, n - o)});
-  const int np = (int)pieces.size();
-  // pieces handed out (-1: stop), their threads, and the shares of the last
-  // one that are not written yet
-  std::atomic<int> ready{0}, workers{0}, left{0};
-  std::vector<std::thread> pool;
-  auto share = [&](int p, int i, int of) {
-    const Piece& q = pieces[p];
-    const size_t b = q.n * i / of, e = q.n * (i + 1) / of;
-    std::memcpy(q.d + b, c->hdata + (p & 1) * half + b, (e - b) * sizeof(double));
-  };
-  auto work = [&](int i) {
-    for (int p = 0; p < np; ++p) {
-      int r;
-      while ((r = ready.load(std::memory_order_acquire)) <= p) {
-        if (r < 0) return;
-        std::this_thread::yield();
-      }
-      share(p, i, workers.load(std::memory_order_relaxed));
-      left.fetch_sub(1, std::memory_order_release);
-    }
-  };
-  try {
-    pool.reserve(HOST_COPY_THREADS);
-    for (int i = 0; i < HOST_COPY_THREADS; ++i) pool.emplace_back(work, i);
-  } catch (const std::exception&) {
-    // as many threads as there are; with none this thread copies
-  }
-  const int nw = (int)pool.size();
-  workers.store(nw, std::memory_order_relaxed);
-  auto drain = [&] {
-    while (left.load(std::memory_order_acquire) > 0) std::this_thread::yield();
-  };
-  hipError_t err = hipSuccess;
-  for (int p = 0; p < np; ++p) {
-    // into the half that piece p - 2 left: it was drained before piece p - 1
-    // was handed out
-    err = hipMemcpyAsync(c->hdata + (p & 1) * half, pieces[p].s, pieces[p].n * sizeof(double), hipMemcpyDeviceToHost,
-                         c->stream);
-    if (err == hipSuccess) err = hipStreamSynchronize(c->stream);
-    if (err != hipSuccess) break;
-    drain();
-    if (nw) {
-      left.store(nw, std::memory_order_relaxed);
-      ready.store(p + 1, std::memory_order_release);
-    } else {
-      share(p, 0, 1);
-    }
-  }
-  drain();
-  if (err != hipSuccess) ready.store(-1, std::memory_order_release);
-  for (auto& t : pool) t.join();
+  const hipError_t err = static_cast<hipError_t>(
+      copy_out(narr, dst, src, n, c->hdata, c->hstage_n / 2, [c](double* to, const double* from, size_t count) -> int {
+        const hipError_t e = hipMemcpyAsync(to, from, count * sizeof(double), hipMemcpyDeviceToHost, c->stream);
+        return e == hipSuccess ? hipStreamSynchronize(c->stream) : e;
+      }));
   HIPCHK(c, err);
   return KB_OK;
 }
