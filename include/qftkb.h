@@ -222,8 +222,9 @@ int kb_reset_timing(kb_ctx *ctx);
 /* ---- tile autotuning -------------------------------------------------------
  * The memory-integral kernel exists in several tile shapes (slot rows per
  * work item, rows per batch, threads per workgroup).  Shape 0, the default,
- * cuts the window into equal runs of rows instead of fixed items in windows
- * of up to 208 steps and where a lattice has few site blocks.  kb_autotune re-times the last step's memory
+ * cuts the window into equal runs of rows instead of fixed items, where that
+ * is faster: in most windows of up to 208 steps and where a lattice has few
+ * site blocks.  kb_autotune re-times the last step's memory
  * integral in every shape (reps launches each, HIP events on the context's
  * stream; each launch recomputes row t from the same inputs, so row t may
  * change in the last bits) and keeps the fastest; ms, if not NULL, receives

@@ -369,10 +369,10 @@ MemintArgs memint_args(const kb_ctx* c) {
   return a;
 }
 
-hipError_t launch_memint(int tile, unsigned grid, int maxN, hipStream_t s, const MemintArgs* args,
+hipError_t launch_memint(int tile, unsigned grid, int maxN, int cus, hipStream_t s, const MemintArgs* args,
                          const int* wg_start, int nruns) {
   // (a table of one run: its arguments are on the device only)
-  if (nruns > 1 && memint_runs_whole(tile, maxN))
+  if (nruns > 1 && memint_runs_whole(tile, maxN, grid, cus))
     return launch_memint_runs(MemintArgs{}, args, wg_start, nruns, grid, maxN, s);
   void* kargs[] = {(void*)&args, (void*)&wg_start, (void*)&nruns};
   return hipLaunchKernel(kMemintVariants[tile].fn, dim3(grid), dim3(kMemintVariants[tile].threads), kargs,
@@ -411,7 +411,7 @@ int launch_memint_step(kb_ctx* c) {
   const MemintArgs a = memint_args(c);
   // (no integrals in the LO expansions: the leapfrog alone, in the item form)
   const bool runs = a.integral && c->tile == 0 && c->rsplit > 1;
-  const bool whole = a.integral && memint_runs_whole(c->tile, c->N);
+  const bool whole = a.integral && memint_runs_whole(c->tile, c->N, c->NB, c->cus);
   const int ns = runs ? c->rsplit : whole ? 1 : c->msplit;
   if (ns > 1) {
     if (runs) {
@@ -429,7 +429,7 @@ int launch_memint_step(kb_ctx* c) {
   }
   hipError_t e = whole
                      ? launch_memint_runs(a, nullptr, nullptr, 1, c->NB, c->N, c->stream)
-                     : launch_memint(c->tile, c->NB, c->N, c->stream, c->margs_dev, c->wg0_dev, 1);
+                     : launch_memint(c->tile, c->NB, c->N, c->cus, c->stream, c->margs_dev, c->wg0_dev, 1);
   if (e != hipSuccess) return seterr(c, KB_ERR_HIP, "memory-integral launch failed: %s", hipGetErrorString(e));
   return KB_OK;
 }
@@ -864,8 +864,7 @@ static int create_ctx(const kb_params* p, bool sym, kb_ctx** out) {
   // this window's LDS size in one round (a grid that overfills some CUs by
   // one workgroup waits for those CUs)
   {
-    int cus = 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, p->device) != hipSuccess ||
+    if (hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, p->device) != hipSuccess ||
         memint_runs_prepare() != hipSuccess)
       return fail(KB_ERR_HIP);
     if (sym) {
@@ -873,9 +872,9 @@ static int create_ctx(const kb_params* p, bool sym, kb_ctx** out) {
       if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)memint_partial<64, 2, 256>, 256,
                                                        memint_lds(c->N)) != hipSuccess)
         return fail(KB_ERR_HIP);
-      c->msplit = std::max(1, std::min(KB_MSPLIT_MAX, per_cu * cus / c->NB));
+      c->msplit = std::max(1, std::min(KB_MSPLIT_MAX, per_cu * c->cus / c->NB));
     }
-    c->rsplit = memint_runs_split(0, c->N, c->NB, cus);
+    c->rsplit = memint_runs_split(0, c->N, c->NB, c->cus);
     const int parts = std::max(c->msplit, c->rsplit);
     if (parts > 1 && (rc = dmalloc(c, (void**)&c->mpart, (size_t)c->NB * parts * 2 * c->N * MB * sizeof(double))))
       return fail(rc);
@@ -1704,7 +1703,7 @@ int ens_enqueue(kb_ens* e) {
     }
     if (rc == KB_OK && e->lane_integrals && e->lwg[j] > 0) {
       // one shape for all members (their item tables follow its row height)
-      err = launch_memint(e->tile, e->lwg[j], e->lmaxN[j], sj, e->margs_dev + e->lrun[j],
+      err = launch_memint(e->tile, e->lwg[j], e->lmaxN[j], e->m[0]->cus, sj, e->margs_dev + e->lrun[j],
                           e->lwg_dev + e->lrun[j], e->lrun[j + 1] - e->lrun[j]);
       if (err != hipSuccess) rc = ens_err(e, KB_ERR_HIP, "memint launch failed: %s", hipGetErrorString(err));
     }
@@ -1720,7 +1719,8 @@ int ens_enqueue(kb_ens* e) {
   }
   if (rc) return rc;
   if (!e->lane_integrals) {
-    err = launch_memint(e->tile, e->total_wg, e->maxN, e->stream, e->margs_dev, e->wg_dev, (int)e->m.size());
+    err = launch_memint(e->tile, e->total_wg, e->maxN, e->m[0]->cus, e->stream, e->margs_dev, e->wg_dev,
+                        (int)e->m.size());
     if (err != hipSuccess) return ens_err(e, KB_ERR_HIP, "memint launch failed: %s", hipGetErrorString(err));
   }
   return KB_OK;
@@ -1823,7 +1823,7 @@ int kb_ens_autotune(kb_ens* e, int reps, int* best, double* ms) {
     for (int k = 0; k <= reps && rc == KB_OK; ++k) {
       if (k == 1 && hipEventRecord(a, e->stream) != hipSuccess) rc = ens_err(e, KB_ERR_HIP, "autotune: event");
       if (rc == KB_OK &&
-          launch_memint(v, e->total_wg, e->maxN, e->stream, e->margs_dev, e->wg_dev, nr) != hipSuccess)
+          launch_memint(v, e->total_wg, e->maxN, e->m[0]->cus, e->stream, e->margs_dev, e->wg_dev, nr) != hipSuccess)
         rc = ens_err(e, KB_ERR_HIP, "autotune: launch failed");
     }
     if (rc) break;

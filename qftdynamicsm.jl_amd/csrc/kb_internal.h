@@ -79,6 +79,7 @@ struct kb_ctx {
   int tile = 0;           // memory-integral tile shape (kMemintVariants index)
   int msplit = 1;         // workgroups per site block of the memory integral (split form if > 1)
   int rsplit = 1;         // the same where tile 0 runs as equal runs
+  int cus = 0;            // of the device
   double* mpart = nullptr;  // their partial accumulators
   int nsplit = 1;           // the same for the 1/N resummation sweeps
   double* npart = nullptr;  // their partial accumulators
@@ -187,7 +188,7 @@ int enqueue_step(kb_ctx* c);
 size_t memint_lds(int N);
 // launch the forward memory-integral kernel of tile shape `tile` on args/wg
 // tables; maxN: the longest of the runs' windows
-hipError_t launch_memint(int tile, unsigned grid, int maxN, hipStream_t s, const qftkb::MemintArgs* args,
+hipError_t launch_memint(int tile, unsigned grid, int maxN, int cus, hipStream_t s, const qftkb::MemintArgs* args,
                          const int* wg_start, int nruns);
 
 // times one stage of kb_timing while in scope

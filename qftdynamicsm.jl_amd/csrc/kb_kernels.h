@@ -221,7 +221,7 @@ __global__ void memint_finish(MemintArgs a, int nsplit, const double* part);
 // up to N; a single run's arguments by value (nruns 1), or the tables of
 // memint_step.  The split form takes memint_runs_split(...) > 1 workgroups
 // per site block, followed by memint_finish.
-bool memint_runs_whole(int tile, int N);
+bool memint_runs_whole(int tile, int N, unsigned blocks, int cus);
 int memint_runs_split(int tile, int N, int NB, int cus);
 hipError_t memint_runs_prepare();
 hipError_t launch_memint_runs(const MemintArgs& one, const MemintArgs* runs, const int* wg_start, int nruns,
