@@ -9,8 +9,8 @@ namespace qftkb {
 namespace {
 
 constexpr int SIGMA_DEVICES = 64;  // (further ones are prepared at every call)
-constexpr int FORMS[] = {FORM_COMPILED, PLAN_SMALL, PLAN_ANY, PLAN_WIDE};
-constexpr int NFORMS = 4, NMODES = SG_PLAIN + 1;
+constexpr int FORMS[] = {FORM_FLAT, FORM_WHOLE, FORM_PASSES, PLAN_SMALL, PLAN_ANY, PLAN_WIDE};
+constexpr int NFORMS = 6, NMODES = SG_PLAIN + 1;
 
 struct FormCode {
   hipError_t (*launch)(const SigmaArgs&, int, int, hipStream_t);
@@ -24,8 +24,9 @@ struct FormCode {
   hipError_t sigma_form<MODE, FORM>(const SigmaArgs&, int rows, int want, hipStream_t st); \
   template <>                                                                          \
   hipError_t sigma_form_prepare<MODE, FORM>();
-#define KB_MODE(MODE) \
-  KB_FORM(MODE, FORM_COMPILED) KB_FORM(MODE, PLAN_SMALL) KB_FORM(MODE, PLAN_ANY) KB_FORM(MODE, PLAN_WIDE)
+#define KB_MODE(MODE)                                                                \
+  KB_FORM(MODE, FORM_FLAT) KB_FORM(MODE, FORM_WHOLE) KB_FORM(MODE, FORM_PASSES)      \
+  KB_FORM(MODE, PLAN_SMALL) KB_FORM(MODE, PLAN_ANY) KB_FORM(MODE, PLAN_WIDE)
 KB_MODE(SG_SUNSET)
 KB_MODE(SG_SUNSET_ADJ)
 KB_MODE(SG_BUBBLE)
@@ -38,8 +39,9 @@ namespace {
 
 // (in the order of SigmaMode and of FORMS)
 #define KB_FORM(MODE, FORM) {sigma_form<MODE, FORM>, sigma_form_prepare<MODE, FORM>}
-#define KB_MODE(MODE) \
-  {KB_FORM(MODE, FORM_COMPILED), KB_FORM(MODE, PLAN_SMALL), KB_FORM(MODE, PLAN_ANY), KB_FORM(MODE, PLAN_WIDE)}
+#define KB_MODE(MODE)                                                                 \
+  {KB_FORM(MODE, FORM_FLAT),  KB_FORM(MODE, FORM_WHOLE), KB_FORM(MODE, FORM_PASSES),  \
+   KB_FORM(MODE, PLAN_SMALL), KB_FORM(MODE, PLAN_ANY),   KB_FORM(MODE, PLAN_WIDE)}
 const FormCode kForms[NMODES][NFORMS] = {KB_MODE(SG_SUNSET), KB_MODE(SG_SUNSET_ADJ), KB_MODE(SG_BUBBLE),
                                          KB_MODE(SG_CHAIN), KB_MODE(SG_PLAIN)};
 #undef KB_MODE
@@ -55,7 +57,7 @@ int form_index(int form) {
 
 void plan_fft(FFTPlan& pl, int n) { pl = make_plan(n); }
 
-// A first call on a device also loads the form's code there (some 1.2 ms per
+// A first call on a device also loads the form's code there (some 2.5 ms per
 // MB: all of it took 13 ms of a process's first kb_create), so only what a
 // lattice runs is prepared.
 hipError_t sigma_prepare(SigmaMode mode, int Nx, int sdim, int device) {

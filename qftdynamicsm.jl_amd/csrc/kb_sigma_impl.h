@@ -1211,8 +1211,9 @@ hipError_t launch_compiled(const SigmaArgs& a, dim3 grid, hipStream_t st) {
 }
 
 // the forms that the code of a mode comes in, each in an object file of its
-// own: FORM_COMPILED, the compiled lengths, and the classes of run-time plans
-constexpr int FORM_COMPILED = 1;
+// own: the compiled lengths, as lines and planes, whole rows or three passes, and
+// the classes of run-time plans
+constexpr int FORM_FLAT = 1, FORM_WHOLE = 2, FORM_PASSES = 3;
 
 constexpr int plan_class(const FFTPlan& pl) {
   int top = 0;
@@ -1226,9 +1227,10 @@ constexpr bool by_whole_rows(int n, int rows) {
 // the form of a stage over `rows` rows
 constexpr int stage_form(const FFTPlan& pl, int sdim, int rows) {
   const int n = pl.n;
-  const bool compiled = sdim == 1 || n == 1 ? row_compiled(n)
-                                            : (sdim == 3 && by_whole_rows(n, rows)) || (planes_fit(n) && n % 8 == 0);
-  return compiled ? FORM_COMPILED : plan_class(pl);
+  if (sdim == 1 || n == 1) return row_compiled(n) ? FORM_FLAT : plan_class(pl);
+  if (sdim == 3 && by_whole_rows(n, rows)) return FORM_WHOLE;
+  if (!planes_fit(n) || n % 8) return plan_class(pl);
+  return sdim == 2 ? FORM_FLAT : FORM_PASSES;
 }
 
 template <int MODE, int KIND, int CLASS>
@@ -1258,19 +1260,23 @@ hipError_t launch_length(const SigmaArgs& a, int n, dim3 grid, hipStream_t st) {
 template <int MODE>
 constexpr int row_last = MODE == SG_PLAIN ? TWIDDLE_MAX : ROW_MAX;
 
-template <int MODE>
+template <int MODE, int FORM>
 hipError_t launch_compiled_stage(const SigmaArgs& a, int rows, hipStream_t st) {
   const int n = a.n;
-  if (a.ny == 1) return launch_length<MODE, KIND_ROW, ROW_MIN, row_last<MODE>, 0>(a, n, dim3(1, rows), st);
-  if (a.nz == 1) return launch_length<MODE, KIND_ALL, 8, 64, 8>(a, n, dim3(1, rows), st);
-  if (by_whole_rows(n, rows)) return launch_length<MODE, KIND_WHOLE, 2, WHOLE_MAX, 1>(a, n, dim3(1, rows), st);
-  const PassPlan last = pass_plan(a.plan, KIND_LAST, true, CT_WANT);
-  const int nh = n / 2 + 1;
-  const dim3 gx(nh, rows), gl(last.tiles * nh, rows);
-  hipError_t e;
-  if ((e = launch_length<MODE, KIND_FWD, SPREAD_MIN, 64, 8>(a, n, gx, st)) != hipSuccess) return e;
-  if ((e = launch_length<MODE, KIND_LAST, SPREAD_MIN, 64, 8>(a, n, gl, st)) != hipSuccess) return e;
-  return launch_length<MODE, KIND_INV, SPREAD_MIN, 64, 8>(a, n, gx, st);
+  if constexpr (FORM == FORM_WHOLE) {
+    return launch_length<MODE, KIND_WHOLE, 2, WHOLE_MAX, 1>(a, n, dim3(1, rows), st);
+  } else if constexpr (FORM == FORM_FLAT) {
+    if (a.ny == 1) return launch_length<MODE, KIND_ROW, ROW_MIN, row_last<MODE>, 0>(a, n, dim3(1, rows), st);
+    return launch_length<MODE, KIND_ALL, 8, 64, 8>(a, n, dim3(1, rows), st);
+  } else {
+    const PassPlan last = pass_plan(a.plan, KIND_LAST, true, CT_WANT);
+    const int nh = n / 2 + 1;
+    const dim3 gx(nh, rows), gl(last.tiles * nh, rows);
+    hipError_t e;
+    if ((e = launch_length<MODE, KIND_FWD, SPREAD_MIN, 64, 8>(a, n, gx, st)) != hipSuccess) return e;
+    if ((e = launch_length<MODE, KIND_LAST, SPREAD_MIN, 64, 8>(a, n, gl, st)) != hipSuccess) return e;
+    return launch_length<MODE, KIND_INV, SPREAD_MIN, 64, 8>(a, n, gx, st);
+  }
 }
 
 // want: threads per workgroup asked for
@@ -1330,14 +1336,18 @@ hipError_t prepare_plan_stage() {
   if (e == hipSuccess) e = prepare_pass<MODE, KIND_LAST, CLASS>();
   return e == hipSuccess ? prepare_pass<MODE, KIND_INV, CLASS>() : e;
 }
-template <int MODE>
+template <int MODE, int FORM>
 hipError_t prepare_compiled_stage() {
-  hipError_t e = prepare_lengths<MODE, KIND_ROW, ROW_MIN, row_last<MODE>, 0>();
-  if (e == hipSuccess) e = prepare_lengths<MODE, KIND_WHOLE, 2, WHOLE_MAX, 1>();
-  if (e == hipSuccess) e = prepare_lengths<MODE, KIND_ALL, 8, 64, 8>();
-  if (e == hipSuccess) e = prepare_lengths<MODE, KIND_FWD, SPREAD_MIN, 64, 8>();
-  if (e == hipSuccess) e = prepare_lengths<MODE, KIND_LAST, SPREAD_MIN, 64, 8>();
-  return e == hipSuccess ? prepare_lengths<MODE, KIND_INV, SPREAD_MIN, 64, 8>() : e;
+  if constexpr (FORM == FORM_WHOLE) {
+    return prepare_lengths<MODE, KIND_WHOLE, 2, WHOLE_MAX, 1>();
+  } else if constexpr (FORM == FORM_FLAT) {
+    const hipError_t e = prepare_lengths<MODE, KIND_ROW, ROW_MIN, row_last<MODE>, 0>();
+    return e == hipSuccess ? prepare_lengths<MODE, KIND_ALL, 8, 64, 8>() : e;
+  } else {
+    hipError_t e = prepare_lengths<MODE, KIND_FWD, SPREAD_MIN, 64, 8>();
+    if (e == hipSuccess) e = prepare_lengths<MODE, KIND_LAST, SPREAD_MIN, 64, 8>();
+    return e == hipSuccess ? prepare_lengths<MODE, KIND_INV, SPREAD_MIN, 64, 8>() : e;
+  }
 }
 
 }  // namespace

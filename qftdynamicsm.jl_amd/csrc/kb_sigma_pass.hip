@@ -8,7 +8,7 @@ namespace qftkb {
 template <>
 hipError_t sigma_form<KB_SIGMA_MODE, KB_SIGMA_FORM>(const SigmaArgs& a, int rows, int want, hipStream_t st) {
 #if KB_SIGMA_COMPILED
-  return launch_compiled_stage<KB_SIGMA_MODE>(a, rows, st);
+  return launch_compiled_stage<KB_SIGMA_MODE, KB_SIGMA_FORM>(a, rows, st);
 #else
   return launch_plan_stage<KB_SIGMA_MODE, KB_SIGMA_FORM>(a, rows, want, st);
 #endif
@@ -17,7 +17,7 @@ hipError_t sigma_form<KB_SIGMA_MODE, KB_SIGMA_FORM>(const SigmaArgs& a, int rows
 template <>
 hipError_t sigma_form_prepare<KB_SIGMA_MODE, KB_SIGMA_FORM>() {
 #if KB_SIGMA_COMPILED
-  return prepare_compiled_stage<KB_SIGMA_MODE>();
+  return prepare_compiled_stage<KB_SIGMA_MODE, KB_SIGMA_FORM>();
 #else
   return prepare_plan_stage<KB_SIGMA_MODE, KB_SIGMA_FORM>();
 #endif
