@@ -184,7 +184,7 @@ def ensemble_bench(args):
         ens.step(t)
         t += 1
     # the pooled memory integral's shape, timed on the last step (then one
-    # step to capture the graph again)
+    # step in it)
     tuned = ens.autotune(3)
     ens.step(t)
     t += 1

@@ -376,7 +376,9 @@ const char *kb_ens_last_error(const kb_ens *ens);
 int kb_ens_member(kb_ens *ens, int i, kb_ctx **member);
 /* Every member takes step t (all members must be at tmax = t - 1). */
 int kb_ens_step(kb_ens *ens, int t);
-/* Capture one ensemble step as a hipGraph and replay it (on = 1). */
+/* Accepted for programs that ask for graph replay; ensemble steps are launched
+ * kernel by kernel all the same (a replayed graph with a branch per stream has
+ * ended processes). */
 int kb_ens_use_graph(kb_ens *ens, int on);
 int kb_ens_synchronize(kb_ens *ens);
 /* HIP-event time of whole ensemble steps since the last reset. */

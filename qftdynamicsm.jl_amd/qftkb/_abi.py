@@ -595,6 +595,7 @@ class KBEnsemble:
         self._chk(self._L.kb_ens_step(self._h, int(t)))
 
     def use_graph(self, on=True):
+        """Accepted; ensemble steps are launched kernel by kernel all the same."""
         self._chk(self._L.kb_ens_use_graph(self._h, 1 if on else 0))
 
     def set_tiles(self, variant):
