@@ -20,7 +20,7 @@
 //      adjoint of step t+1 into F_bar(t,t);
 //   3. adj_reduce_kernel: the self-energy adjoints Sigma_bar of the memory
 //      integrals, reduced per slot in LDS from one read of H;
-//   4. the self-energy stage run backwards (kb_sigma.hip, ADJ) adds the
+//   4. the self-energy stage run backwards (SG_SUNSET_ADJ) adds the
 //      sunset adjoint into row t-1 of Hbar;
 //   5. every AK (8) reverse steps, adj_apply_kernel adds the memory integrals'
 //      entry adjoints of those steps to Hbar in one read-modify-write

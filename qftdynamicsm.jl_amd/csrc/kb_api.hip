@@ -20,15 +20,15 @@
 #ifndef KB_MSPLIT_MAX
 #define KB_MSPLIT_MAX 8
 #endif
-// largest orbit count whose self-energy runs as orbit products (the matrix
-// takes orbits^2 doubles: 134 MB at the limit)
-// lattice limits: the pencil passes hold two buffers of Nx complex values per
-// pencil in LDS (64 KiB at Nx = 2048, one pencil per workgroup); with at most
-// 2^24 sites a launch of one workgroup per 8-site block stays below 2^32
-// work-items at 1024 threads per workgroup
+// lattice limits: a transform pass holds its lines and Nx twiddles in LDS (131
+// KB at Nx = 2048, three lines per workgroup); with at most 2^24 sites a launch
+// of one workgroup per 8-site block stays below 2^32 work-items at 1024 threads
+// per workgroup
 constexpr int KB_MAX_NX = 2048;
 constexpr long KB_MAX_SITES = 1L << 24;
 
+// largest orbit count whose self-energy runs as orbit products (the matrix
+// takes orbits^2 doubles: 134 MB at the limit)
 #ifndef KB_ORBIT_PRODUCT_MAX
 #define KB_ORBIT_PRODUCT_MAX 4096
 #endif

@@ -145,8 +145,9 @@ struct kb_ctx {
 namespace qftkb_host {
 
 int seterr(kb_ctx* c, int code, const char* fmt, ...);
-// the twiddles exp(-2 pi i k / n), k < n (long double on the host), shared by
-// contexts and the context-free entry points
+// the twiddles exp(-2 pi i k / n), k < n, of a context: up to 64 the table of
+// kb_twiddles.h, which the context-free entry points use too, beyond it rounded
+// from long double
 void fft_twiddles(int n, double2* out);
 // message of the calling thread's last failed context-free call
 const char* free_call_error();

@@ -68,7 +68,7 @@ __host__ __device__ inline StepState state_of_step(int t, int N) {
   return s;
 }
 
-// modes of the plane kernels (kb_sigma.hip)
+// modes of the self-energy stage (kb_sigma_impl.h)
 // SG_PLAIN is the sunset of caller-supplied lattices: rows q < rows of the
 // physical F and rho in Fin/Rin (q * V + site), Sigma into SigFout/Sigrout
 enum SigmaMode { SG_SUNSET = 0, SG_SUNSET_ADJ = 1, SG_BUBBLE = 2, SG_CHAIN = 3, SG_PLAIN = 4 };

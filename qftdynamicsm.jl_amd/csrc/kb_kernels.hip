@@ -518,8 +518,8 @@ __global__ __launch_bounds__(MEMINT_FINISH_THREADS) void memint_finish(MemintArg
 // while its first rows are on their way; one row (4 lines) is in flight per
 // worker: 2 or 3 need more than 128 registers, and fewer waves cost more
 // than the deeper pipeline gives.
-// Measured (64-row items -> runs): 112^3 N_mem = 16 4868 -> 906 us (0.63 ->
-// 3.4 TB/s), 64^3 N_mem = 32 1267 -> 544 us, 48^3 N_mem = 48 742 -> 466 us,
+// Measured (64-row items -> runs): 112^3 N_mem = 16 4868 -> 946 us (0.63 ->
+// 3.2 TB/s), 64^3 N_mem = 32 1267 -> 544 us, 48^3 N_mem = 48 742 -> 466 us,
 // 42^3 N_mem = 96 1146 -> 1085 us (5.1 TB/s), 32^3 N_mem = 150 1111 -> 1043
 // us (5.7 TB/s), 16^3 N_mem = 64 37.6 -> 30.6 us, 16^2 N_mem = 24 13.3 -> 6.4
 // us.  Past N_mem = 208 the staged items are as fast (32^3 N_mem = 300: 3840
@@ -792,7 +792,10 @@ __global__ __launch_bounds__(TPB, D > 1 ? 3 : 4) void memint_partial_runs(Memint
 
 constexpr int RUNS_MAX_N = 208;       // longest window of the whole-block form
 constexpr int RUNS_FOUR_MAX_N = 152;  // longest of which four workgroups fit a CU (256 bytes of LDS per slot)
-constexpr int RUNS_SPLIT_MIN_N = 48;  // shorter windows: the second launch costs more than it gives
+// Shorter windows: the second launch costs more than the split gives.  A step of
+// 8^3 whole and split: N_mem 40 19.8 and 21.3 us, 48 20.7 and 22.4, 56 24.4 and
+// 23.0, 64 28.2 and 23.5, 100 50.5 and 28.9 (the two are level at some 52).
+constexpr int RUNS_SPLIT_MIN_N = 48;
 constexpr int RUNS_SPLIT_MAX_N = 600; // 256 bytes of LDS per slot
 constexpr int RUNS_SPLIT_THREADS = 512;
 

@@ -90,7 +90,10 @@ size_t sigma_workspace_values(int Nx, int sdim, size_t rows) {
 // whose stage serves orbit storage through its site maps
 bool sigma_planes_supported(int Nx, int sdim) { return Nx >= 1 && Nx <= (sdim == 1 ? 2048 : 64); }
 
-// threads per workgroup the autotuner asks for; entry 0 is the default
+// threads per workgroup the autotuner asks for (run-time plans of planes and
+// batches); entry 0 is the default.  A step's stage with 24 rows, us, for 256,
+// 128 and 512: 27^3 34 34 34, 35^3 39 48 39, 45^3 54 70 53, 50^3 65 73 76, 46^3
+// 116 122 137, 57^3 146 133 151, 63^3 128 131 113, 61^3 275 297 201.
 const int kFFTThreads[NFFT_VARIANTS] = {256, 128, 512, 1024};
 
 hipError_t launch_sigma_stage(const SigmaArgs& a, SigmaMode mode, int rows, hipStream_t st, int variant) {
