@@ -198,7 +198,7 @@ int launch_sigma(kb_ctx* c, double2* X, double* S_out) {
     return KB_OK;
   }
   if (plane_workspace_missing(c)) return seterr(c, KB_ERR_STATE, "self-energy: plane workspace not allocated");
-  hipError_t e = launch_sigma_stage(a, SG_SUNSET, L, c->stream, c->fft_tile);
+  hipError_t e = launch_sigma_stage(a, SG_SUNSET, L, c->stream, c->fft_tile, !c->in_ensemble);
   if (e != hipSuccess) return seterr(c, KB_ERR_HIP, "self-energy launch failed: %s", hipGetErrorString(e));
   return KB_OK;
 }
@@ -247,7 +247,7 @@ int launch_bubble(kb_ctx* c, const StepState* st, bool keep) {
   SigmaArgs a = ninv_sigma_args(c, st);
   a.preF = a.preR = ivol * ivol;
   a.X = keep ? c->Xn : nullptr;
-  hipError_t e = launch_sigma_stage(a, SG_BUBBLE, c->N - 1, c->stream);
+  hipError_t e = launch_sigma_stage(a, SG_BUBBLE, c->N - 1, c->stream, 0, !c->in_ensemble);
   if (e != hipSuccess) return seterr(c, KB_ERR_HIP, "bubble launch failed: %s", hipGetErrorString(e));
   return KB_OK;
 }
@@ -301,7 +301,7 @@ int launch_chain(kb_ctx* c) {
   SigmaArgs a = ninv_sigma_args(c, c->st_dev);
   a.preF = a.preR = pre;
   a.X = c->Xn;
-  hipError_t e = launch_sigma_stage(a, SG_CHAIN, c->N - 1, c->stream);
+  hipError_t e = launch_sigma_stage(a, SG_CHAIN, c->N - 1, c->stream, 0, !c->in_ensemble);
   if (e != hipSuccess) return seterr(c, KB_ERR_HIP, "chain launch failed: %s", hipGetErrorString(e));
   return KB_OK;
 }

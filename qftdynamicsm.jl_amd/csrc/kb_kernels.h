@@ -271,7 +271,9 @@ hipError_t sigma_prepare(SigmaMode mode, int Nx, int sdim, int device);
 // variant: index into kFFTThreads (threads per workgroup asked for)
 constexpr int NFFT_VARIANTS = 4;
 extern const int kFFTThreads[NFFT_VARIANTS];
-hipError_t launch_sigma_stage(const SigmaArgs& a, SigmaMode mode, int rows, hipStream_t st, int variant = 0);
+// alone: no other run's stages beside this one's (contexts outside ensembles)
+hipError_t launch_sigma_stage(const SigmaArgs& a, SigmaMode mode, int rows, hipStream_t st, int variant = 0,
+                              bool alone = true);
 
 // self-energy stage of a cubic-orbit-stored window as two FP64 matrix
 // products with the orbit cosine matrix Mo (kb_orbit.hip)

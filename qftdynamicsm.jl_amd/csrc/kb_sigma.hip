@@ -66,7 +66,7 @@ hipError_t sigma_prepare(SigmaMode mode, int Nx, int sdim, int device) {
   bool used[NFORMS] = {};
   if (Nx > 0) {
     const FFTPlan pl = make_plan(Nx);
-    for (int rows : {1, SPREAD_ROWS}) used[form_index(stage_form(pl, sdim, rows))] = true;
+    for (int rows : {1, SPREAD_ROWS}) used[form_index(stage_form(pl, sdim, rows, true))] = true;
   }
   std::lock_guard<std::mutex> lk(mu);
   const bool known = device >= 0 && device < SIGMA_DEVICES;
@@ -96,8 +96,8 @@ bool sigma_planes_supported(int Nx, int sdim) { return Nx >= 1 && Nx <= (sdim ==
 // 116 122 137, 57^3 146 133 151, 63^3 128 131 113, 61^3 275 297 201.
 const int kFFTThreads[NFFT_VARIANTS] = {256, 128, 512, 1024};
 
-hipError_t launch_sigma_stage(const SigmaArgs& a, SigmaMode mode, int rows, hipStream_t st, int variant) {
-  const int form = stage_form(a.plan, a.ny == 1 ? 1 : a.nz == 1 ? 2 : 3, rows);
+hipError_t launch_sigma_stage(const SigmaArgs& a, SigmaMode mode, int rows, hipStream_t st, int variant, bool alone) {
+  const int form = stage_form(a.plan, a.ny == 1 ? 1 : a.nz == 1 ? 2 : 3, rows, alone);
   return kForms[mode][form_index(form)].launch(a, rows, kFFTThreads[variant], st);
 }
 

@@ -665,7 +665,9 @@ constexpr int WHOLE_MAX = 26;
 // that have no compiled passes change over earlier: 25^3 22 against 29 us for 1
 // row, 28 against 30 for 32, 32 against 31 for 48; 26^3 32 against 42, 38
 // against 44, 42 against 45.  (Below 24 whole rows win there from the first
-// row on: 22^3 28 against 32 us, 20^3 18 against 27.)
+// row on: 22^3 28 against 32 us, 20^3 18 against 27.)  Beside other runs' stages,
+// in an ensemble, these stay whole: the chip is filled and launches count (a step
+// of six runs around 20^3, one of them 25^3, with N_mem = 9 104 against 111 us).
 constexpr int ROW_MIN = 8, ROW_MAX = 1024;  // compiled lines: powers of two
 constexpr int SPREAD_MIN = 24, SPREAD_ROWS = 96, SPREAD_PLAN_ROWS = 40;
 // lines along z that stand for themselves and their reflection (-x, -y)
@@ -1221,14 +1223,15 @@ constexpr int plan_class(const FFTPlan& pl) {
   return top <= SMALL_RADIX ? PLAN_SMALL : wide(pl) ? PLAN_WIDE : PLAN_ANY;
 }
 constexpr bool row_compiled(int n) { return n >= ROW_MIN && n <= ROW_MAX && (n & (n - 1)) == 0; }
-constexpr bool by_whole_rows(int n, int rows) {
-  return whole_fits(n) && (n < SPREAD_MIN || rows >= (n % 8 ? SPREAD_PLAN_ROWS : SPREAD_ROWS));
+constexpr bool by_whole_rows(int n, int rows, bool alone) {
+  if (!whole_fits(n)) return false;
+  return n < SPREAD_MIN || (n % 8 ? !alone || rows >= SPREAD_PLAN_ROWS : rows >= SPREAD_ROWS);
 }
-// the form of a stage over `rows` rows
-constexpr int stage_form(const FFTPlan& pl, int sdim, int rows) {
+// the form of a stage over `rows` rows; alone: no other run's stages beside it
+constexpr int stage_form(const FFTPlan& pl, int sdim, int rows, bool alone) {
   const int n = pl.n;
   if (sdim == 1 || n == 1) return row_compiled(n) ? FORM_FLAT : plan_class(pl);
-  if (sdim == 3 && by_whole_rows(n, rows)) return FORM_WHOLE;
+  if (sdim == 3 && by_whole_rows(n, rows, alone)) return FORM_WHOLE;
   if (!planes_fit(n) || n % 8) return plan_class(pl);
   return sdim == 2 ? FORM_FLAT : FORM_PASSES;
 }

@@ -73,3 +73,23 @@ def test_one_row_of_25_takes_no_longer_than_one_of_27():
         ratios.append(best[0] / best[1])
     print(f"\n[case] one row of 25^3 over one of 27^3: {min(ratios):.2f}", flush=True)
     assert min(ratios) <= 1.0  # (whole in one workgroup: 1.1)
+
+
+@pytest.mark.parametrize("Nx", [24, 25, 26])
+def test_ensemble_member_has_the_bits_of_a_lone_run(Nx):
+    """(25^3 and 26^3 stay whole beside other runs)"""
+    from qftkb import KBContext, KBEnsemble
+    print(f"\n[case] ensemble member {Nx}^3", flush=True)
+    args = [dict(Nx=n, sdim=3, NstepsinMemory=7, dt=0.1, Lambda=1.3, ONgroup=2, Mass=1.0, Mass2=1.0) for n in (Nx, 12)]
+    e, c = KBEnsemble(args), KBContext(**args[0])
+    n = np.random.default_rng(Nx).uniform(0.1, 2.0, Nx ** 3)
+    c.fill_free_window(8, n, 1.0)
+    e.members[0].fill_free_window(8, n, 1.0)
+    e.members[1].fill_free_window(8, np.ones(12 ** 3), 1.0)
+    c.step(9)
+    e.step(9)
+    for tp in range(c.window()[0], 9):
+        for w in "Fr":
+            assert np.array_equal(e.members[0].sigma(w, tp), c.sigma(w, tp)), (w, tp)
+    e.close()
+    c.close()
