@@ -373,7 +373,7 @@ hipError_t launch_memint(int tile, unsigned grid, int maxN, int cus, hipStream_t
                          const int* wg_start, int nruns) {
   // (a table of one run: its arguments are on the device only)
   if (nruns > 1 && memint_runs_whole(tile, maxN, grid, cus))
-    return launch_memint_runs(MemintArgs{}, args, wg_start, nruns, grid, maxN, s);
+    return launch_memint_runs(MemintArgs{}, args, wg_start, nruns, grid, maxN, cus, s);
   void* kargs[] = {(void*)&args, (void*)&wg_start, (void*)&nruns};
   return hipLaunchKernel(kMemintVariants[tile].fn, dim3(grid), dim3(kMemintVariants[tile].threads), kargs,
                          memint_lds(maxN), s);
@@ -428,7 +428,7 @@ int launch_memint_step(kb_ctx* c) {
     return KB_OK;
   }
   hipError_t e = whole
-                     ? launch_memint_runs(a, nullptr, nullptr, 1, c->NB, c->N, c->stream)
+                     ? launch_memint_runs(a, nullptr, nullptr, 1, c->NB, c->N, c->cus, c->stream)
                      : launch_memint(c->tile, c->NB, c->N, c->cus, c->stream, c->margs_dev, c->wg0_dev, 1);
   if (e != hipSuccess) return seterr(c, KB_ERR_HIP, "memory-integral launch failed: %s", hipGetErrorString(e));
   return KB_OK;

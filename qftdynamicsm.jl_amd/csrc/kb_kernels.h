@@ -225,7 +225,7 @@ bool memint_runs_whole(int tile, int N, unsigned blocks, int cus);
 int memint_runs_split(int tile, int N, int NB, int cus);
 hipError_t memint_runs_prepare();
 hipError_t launch_memint_runs(const MemintArgs& one, const MemintArgs* runs, const int* wg_start, int nruns,
-                              unsigned grid, int N, hipStream_t s);
+                              unsigned grid, int N, int cus, hipStream_t s);
 hipError_t launch_memint_runs_split(const MemintArgs& a, int NB, int nsplit, double* part, hipStream_t s);
 
 // memory-integral tile shapes: ROWS slot rows per work item, B rows per

@@ -791,6 +791,7 @@ __global__ __launch_bounds__(TPB, D > 1 ? 3 : 4) void memint_partial_runs(Memint
 }
 
 constexpr int RUNS_MAX_N = 208;       // longest window of the whole-block form
+constexpr int LDS_PER_CU = 160 * 1024;
 constexpr int RUNS_FOUR_MAX_N = 152;  // longest of which four workgroups fit a CU (256 bytes of LDS per slot)
 // Shorter windows: the second launch costs more than the split gives.  A step of
 // 8^3 whole and split: N_mem 40 19.8 and 21.3 us, 48 20.7 and 22.4, 56 24.4 and
@@ -799,15 +800,20 @@ constexpr int RUNS_SPLIT_MIN_N = 48;
 constexpr int RUNS_SPLIT_MAX_N = 600; // 256 bytes of LDS per slot
 constexpr int RUNS_SPLIT_THREADS = 512;
 
+// the share of the chip's slots that `blocks` workgroups use over their rounds,
+// in percent
+inline unsigned rounds_full(unsigned blocks, unsigned slots) {
+  const unsigned rounds = (blocks + slots - 1) / slots;
+  return rounds <= 1 ? 100 : 100ull * blocks / ((unsigned long long)rounds * slots);
+}
+
 // Three workgroups to a CU are enough to be faster than the items (six to a CU)
 // unless the blocks' last round leaves most of the slots empty: 1000 blocks on
 // 768 slots took 427 us at N_mem = 192 against 408, 729 blocks (all at once)
 // 285 against 311, 1331 and more 0.89 to 1.02 of the items' time (160 to 208).
 // With four they are faster whatever the number of blocks.
 bool memint_runs_whole(int tile, int N, unsigned blocks, int cus) {
-  if (tile != 0 || N > RUNS_MAX_N) return false;
-  const unsigned slots = 3 * cus, rounds = (blocks + slots - 1) / slots;
-  return N <= RUNS_FOUR_MAX_N || rounds <= 1 || 10 * blocks >= 7 * rounds * slots;
+  return tile == 0 && N <= RUNS_MAX_N && (N <= RUNS_FOUR_MAX_N || rounds_full(blocks, 3 * cus) >= 70);
 }
 
 // Workgroups per site block: one per CU in all.  16^2 and 1D lattices, and
@@ -824,20 +830,23 @@ hipError_t memint_runs_prepare() {
                              hipFuncAttributeMaxDynamicSharedMemorySize, RUNS_SPLIT_MAX_N * 32 * MB);
 }
 
-// Threads per site block: a wave up to N_mem = 32 and two up to 64, if the
-// blocks fill the CUs that way (2048 of them), and two up to 152 from ten blocks
-// per CU on; four otherwise, and eight for long windows on fewer than two blocks
-// per CU (256 blocks, N_mem = 200: 149 us at 256 threads, 121 at 512).  In parts
-// of the items' time, two waves and four: 32^3 N_mem = 48 0.64 both, 100 0.88
-// and 0.90, 150 0.91 and 0.92, but 160 1.02 and 0.94, 192 1.04 and 0.97 (three
-// workgroups of two waves leave a CU idle); on 2048 blocks (128^2) 100 1.04 and
-// 0.94, on 2197 (26^3) 140 1.05 and 0.95.
+// Threads per site block: a wave up to N_mem = 32 and two up to 152, if the
+// blocks fill the CUs that way (2048 of them), two only if their rounds on the
+// chip are at least 80% full (65% up to N_mem = 64; a CU holds eight such
+// workgroups or what its LDS takes); four otherwise, and eight for long windows
+// on fewer than two blocks per CU (256 blocks, N_mem = 200: 149 us at 256
+// threads, 121 at 512).  In parts of the items' time, two waves and four: 40^3
+// N_mem = 48 0.58 and 0.61, 100 0.91 and 0.93, 160 (three to a CU) 1.04 and
+// 0.96; 26^3 112 (86% full) 0.87 and 0.91, 140 (72%) 1.05 and 0.95; 128^2 100
+// (67%) 1.04 and 0.94, 128 (100%) 0.89 and 0.91; 28^3 112 (71%) 0.95 and 0.88,
+// 128 (89%) both 0.89; 160^2 48 (78%) 0.61 and 0.64, 128 (78%) 0.94 and 0.91.
 hipError_t launch_memint_runs(const MemintArgs& one, const MemintArgs* runs, const int* wg_start, int nruns,
-                              unsigned grid, int N, hipStream_t s) {
+                              unsigned grid, int N, int cus, hipStream_t s) {
   const size_t lds = sizeof(double) * 4 * (size_t)N * MB;
   if (grid >= 2048 && N <= 32)
     hipLaunchKernelGGL((memint_step_runs<1, 64, true>), dim3(grid), dim3(64), 2 * lds, s, one, runs, wg_start, nruns);
-  else if (N <= 64 ? grid >= 2048 : N <= RUNS_FOUR_MAX_N && grid >= 2560)
+  else if (grid >= 2048 && N <= RUNS_FOUR_MAX_N &&
+           rounds_full(grid, cus * min(8, LDS_PER_CU / (int)(lds + 256))) >= (N <= 64 ? 65 : 80))
     hipLaunchKernelGGL((memint_step_runs<1, 128, false>), dim3(grid), dim3(128), lds, s, one, runs, wg_start, nruns);
   else if (grid >= 512 || N < 128)
     hipLaunchKernelGGL((memint_step_runs<1, 256, false>), dim3(grid), dim3(256), lds, s, one, runs, wg_start, nruns);

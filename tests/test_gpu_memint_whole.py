@@ -1,8 +1,8 @@
 """The equal-run memory integral of whole site blocks at the limits of its
 forms (site blocks enough that none is split: eight waves per block and four
-from 512 blocks on, two from 2048 on up to N_mem = 64 and from 2560 on up to
-152, the longest window of 208, the item form where the last round would be
-nearly empty), for one run and for an ensemble's table, against the item form
+from 512 blocks on, two from 2048 on up to N_mem = 152 where their rounds fill
+the chip, the longest window of 208, the item form where the
+last round would be nearly empty), for one run and for an ensemble's table, against the item form
 of the same integrals (shape 1, tested against the oracle), through a wrapped
 ring; tolerance 1e-10, norm-wise relative."""
 import numpy as np
@@ -27,9 +27,9 @@ def same_row(a, b, t):
 
 
 # 422 site blocks: eight waves from N_mem = 128 to 208; 512: four; 1000: four, items
-# from 153 on; 2197: two up to 64; 2744: two up to 152
+# from 153 on; 2197: four at 64 (two at 112); 2744: two at 128 and 152
 @pytest.mark.parametrize("Nx,N", [(15, 127), (15, 128), (15, 208), (15, 209), (16, 202), (16, 208), (20, 152),
-                                  (20, 153), (26, 64), (26, 65), (26, 192), (26, 193), (28, 152), (28, 153)])
+                                  (20, 153), (26, 64), (26, 112), (26, 192), (26, 193), (28, 128), (28, 152), (28, 153)])
 def test_whole_blocks_match_items(Nx, N):
     from qftkb import KBContext
     print(f"\n[case] whole blocks {Nx}^3 N_mem={N}", flush=True)
@@ -46,10 +46,10 @@ def test_whole_blocks_match_items(Nx, N):
         c.close()
 
 
-# 3000 site blocks: one wave up to N_mem = 32, two to 152, four past it (2729);
-# 895: four, items from 153 on; 281: eight past 127
-@pytest.mark.parametrize("sizes,N", [((20, 20, 20), 24), ((20, 20, 20), 33), ((20, 20, 20), 64), ((16, 12, 11), 64),
-                                     ((16, 12, 11), 130), ((16, 12, 11), 160), ((9, 8, 10), 130), ((20, 18, 20), 153),
+# 3000 site blocks: one wave up to N_mem = 32, two at 33, 64 and 112; 2729: four past
+# 152; 895: four, items from 153 on; 281: eight past 127
+@pytest.mark.parametrize("sizes,N", [((20, 20, 20), 24), ((20, 20, 20), 33), ((20, 20, 20), 64),
+                                     ((20, 20, 20), 112), ((16, 12, 11), 64), ((16, 12, 11), 130), ((16, 12, 11), 160), ((9, 8, 10), 130), ((20, 18, 20), 153),
                                      ((20, 18, 20), 193)])
 def test_tables_match_items(sizes, N):
     from qftkb import KBContext, KBEnsemble
