@@ -57,9 +57,9 @@ int form_index(int form) {
 
 void plan_fft(FFTPlan& pl, int n) { pl = make_plan(n); }
 
-// A first call on a device also loads the form's code there (some 2.5 ms per
-// MB: all of it took 13 ms of a process's first kb_create), so only what a
-// lattice runs is prepared.
+// A first call on a device also loads the form's code there (1 to 2 ms; all of it
+// took 13 ms of a process's first kb_create), so only what a lattice runs is
+// prepared.
 hipError_t sigma_prepare(SigmaMode mode, int Nx, int sdim, int device) {
   static std::mutex mu;
   static bool ready[SIGMA_DEVICES][NMODES][NFORMS] = {};
